@@ -1,33 +1,36 @@
 // rw_attn.hpp -- multi-head attention on gfx950 (device code).
 //
 // out[t_q, n_state] = concat_h softmax(q_h k_h^T / sqrt(64) + mask) v_h, as
-// mha_split_kv (src/encoder.rs:48-80) computes it in f32.  Two launches:
+// mha_split_kv (src/encoder.rs:48-80) computes it in f32.
 //
-//   k_attn_split   q, k and v (f32) -> f16 pairs, one launch
-//        x = hi + lo (hi = f16(x), lo = f16(x - hi)), head-major planes:
-//        q, k  [head][t_pad][64]      (q pre-scaled by 1/8, exact)
-//        v^T   [head][64][t_kv_pad]   kv positions permuted in 16-blocks
-//   k_attn    one workgroup per (64 query rows, head), two wavefronts that
-//        split the kv blocks between them and meet in LDS at the end.
+//   k_attn_split   k and v (f32) -> f16 pairs x = hi + lo (hi = f16(x), lo =
+//        f16(x - hi)), stored as the matrix cores' operands: per (head, 32 kv
+//        rows) the 16 KB of ATT_BLK below
+//   k_attn_tile    calls of more than 8 query rows: one workgroup per (32 or
+//        64 query rows, head), whose 4 wavefronts split the kv blocks
+//        between them and meet in LDS at the end
+//   k_attn    calls of at most 8 query rows (a decoding step): one workgroup of
+//        two wavefronts per (head[, kv run])
 //
 // Precision.  Every product runs on v_mfma_f32_32x32x16_f16 as three f16
 // products, hi*hi + hi*lo + lo*hi, accumulated in f32: each operand keeps
 // 22 of f32's 24 significant bits and the dropped lo*lo term is below 2^-22
 // of the product, so outputs stay within about 1e-6 (relative to the row) of
 // the exact result, like the reference's f32 arithmetic.  Probabilities
-// enter as 2^12 p so that small ones keep their f16 bits.  Inputs must stay
-// below f16's 65504 in magnitude (whisper's projections are far below it);
-// inputs below about 1e-3 lose a few bits to f16 subnormal residuals.  The
-// softmax is online (running maximum and sum per query row, rescaled per
-// block) in f32, which is the reference's max / exp / sum / divide reordered.
+// enter scaled by 2^8 or more (ATT_PS) so that small ones keep their f16 bits.
+// Inputs must stay below f16's 65504 in magnitude (whisper's projections are
+// far below it); inputs below about 1e-3 lose a few bits to f16 subnormal
+// residuals.  The softmax is online (running reference exponent and sum per
+// query row) in f32, which is the reference's max / exp / sum / divide
+// reordered.
 //
-// Layouts inside k_attn.  The score block is computed transposed, S^T = K Q^T
-// (32 kv x 32 queries): lane (h, n) then holds 16 kv entries of query n, so a
+// Layouts inside the kernels.  The score block is computed transposed, S^T =
+// K Q^T (32 kv x 32 queries): lane (h, n) then holds 16 kv entries of query n, so a
 // query row's maximum and sum are in-lane plus one exchange with lane n+32.
 // The output is accumulated transposed as well, O^T = V^T P^T, so the
 // per-block rescale of a query column is one multiplier per lane.  P^T's
 // registers feed that MFMA's B operand directly: lane half h holds kv
-// 4h..4h+3 and 8+4h..8+4h+3 of each 16, and the v^T plane stores each
+// 4h..4h+3 and 8+4h..8+4h+3 of each 16, and the v^T operands hold each
 // 16-block of kv positions in that order (attn_vpos).
 #pragma once
 #include <stdint.h>
@@ -38,23 +41,35 @@ namespace rw {
 
 constexpr int ATT_DH = 64;   // head size (every whisper model)
 constexpr int ATT_KVB = 32;  // kv rows per block
-constexpr int ATT_QT = 2;    // 32-query tiles per workgroup
-constexpr int ATT_QB = 32 * ATT_QT;
+constexpr int ATT_QB = 64;   // query rows a workspace's rows are padded to
+constexpr int ATT_NK = 4;    // wavefronts of a k_attn_tile workgroup
+constexpr int ATT_STEP_MAX = 8;   // query rows of a k_attn call at most
+constexpr int ATT_ROWS_MAX = 64;  // query rows of a call that splits K and V as it loads them, at most
 #ifndef ATT_MAX_SPLIT_N
 #define ATT_MAX_SPLIT_N 32
 #endif
 constexpr int ATT_MAX_SPLIT = ATT_MAX_SPLIT_N;  // kv runs of one (query block, head) at most
 static_assert(ATT_MAX_SPLIT < 128, "k_attn packs the run count into 7 bits");
 
-// kv index (within a 16-block) stored at position p of the v^T plane: the
+// kv index (within a 16-block) stored at position p of the v^T operands: the
 // middle quads swap (an involution)
 RW_HD inline int attn_vpos(int p) {
   const int qd = (p >> 2) & 3;
   return qd == 1 ? p + 4 : qd == 2 ? p - 4 : p;
 }
 
+// K and v^T of one (head, 32 kv rows) as operands: four parts of ATT_PART
+// f16 (K hi, K lo, v^T hi, v^T lo), each 4 fragments [64 lanes][8], so that a
+// wavefront's load of a fragment is one contiguous 1 KB.  K's fragment s:
+// lane 32 h + n holds values 16 s + 8 h .. + 7 of kv row n.  v^T's fragment
+// 2 dt + s: lane 32 h + n holds value 32 dt + n of kv rows 16 s + attn_vpos(8 h
+// + e), e = 0 .. 7.  (Row-major planes, whose lanes read 16-byte pieces 128
+// bytes apart, held the large-v3 encoder's attention at 62 us.)
+constexpr int ATT_PART = 4 * 64 * 8;
+constexpr int ATT_BLK = 4 * ATT_PART;  // f16 per (head, block)
+
 struct AttnPlanes {
-  const uint16_t *qh, *ql, *kh, *kl, *vh, *vl;
+  const uint16_t *kv;  // [head][tkv_pad / 32][ATT_BLK]
   int tq_pad, tkv_pad;
 };
 
@@ -63,8 +78,12 @@ struct AttnPlanes {
 typedef _Float16 att_v8h __attribute__((ext_vector_type(8)));
 typedef float att_v16f __attribute__((ext_vector_type(16)));
 
+typedef float att_v2f __attribute__((ext_vector_type(2)));
+typedef _Float16 att_v2h __attribute__((ext_vector_type(2)));
+constexpr float ATT_LOG2E = 1.4426950408889634f;
+constexpr float ATT_STEP_PS = 4096.0f;  // k_attn's scale of P
+
 // x = hi + lo, both f16
-constexpr float ATT_PS = 4096.0f;
 __device__ inline void att_split(float x, uint16_t &hi, uint16_t &lo) {
   const _Float16 h = (_Float16)x;
   const _Float16 l = (_Float16)(x - (float)h);
@@ -72,93 +91,49 @@ __device__ inline void att_split(float x, uint16_t &hi, uint16_t &lo) {
   lo = __builtin_bit_cast(uint16_t, l);
 }
 
-// q or k rows -> [head][t_pad][64] f16 pairs; rows >= t are zeros.  Item
-// idx covers 8 consecutive values of one row and head.
-__device__ inline void att_split_rows(size_t idx, const float *__restrict__ x, int ld, int t, int t_pad,
-                                      float scale, uint16_t *__restrict__ hi, uint16_t *__restrict__ lo) {
-  const int c = (int)(idx & 7);
-  const size_t hr = idx >> 3;  // head * t_pad + row
-  const int row = (int)(hr % t_pad), head = (int)(hr / t_pad);
-  float v[8];
-  if (row < t) {
-    const float4 *src = reinterpret_cast<const float4 *>(x + (size_t)row * ld + head * ATT_DH + c * 8);
-    const float4 a = src[0], b = src[1];
-    v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
-  } else {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = 0.0f;
-  }
+// 8 f32 values -> the 8 hi and the 8 lo halves
+__device__ inline void att_split8(const float (&v)[8], uint16_t *__restrict__ hi, uint16_t *__restrict__ lo) {
   uint16_t h8[8], l8[8];
 #pragma unroll
-  for (int e = 0; e < 8; ++e) att_split(v[e] * scale, h8[e], l8[e]);
-  const size_t o = hr * ATT_DH + c * 8;
-  *reinterpret_cast<uint4 *>(hi + o) = *reinterpret_cast<const uint4 *>(h8);
-  *reinterpret_cast<uint4 *>(lo + o) = *reinterpret_cast<const uint4 *>(l8);
+  for (int e = 0; e < 8; ++e) att_split(v[e], h8[e], l8[e]);
+  *reinterpret_cast<uint4 *>(hi) = *reinterpret_cast<const uint4 *>(h8);
+  *reinterpret_cast<uint4 *>(lo) = *reinterpret_cast<const uint4 *>(l8);
 }
 
-// v^T [head][64][t_pad] f16 pairs: kv positions permuted by attn_vpos within
-// each 16-block; kv >= t are zeros.
-// v -> v^T pairs, one workgroup per (head, 64 kv positions): the 64 x 64
-// values are read as row-contiguous 16-byte loads, split, and transposed
-// through LDS (each position at its attn_vpos place, an involution), then
-// written as 128-byte runs of positions per d and plane.  `sh` holds 2 x 64
-// rows of ATT_VT_LD halves.
-constexpr int ATT_VT_KV = 64, ATT_VT_LD = ATT_VT_KV + 8;
-__device__ inline int att_vt_tiles(int t_pad) { return (t_pad + ATT_VT_KV - 1) / ATT_VT_KV; }
-__device__ inline void att_split_vt_tile(int tile, const float *__restrict__ v, int ld, int t, int t_pad,
-                                         uint16_t *__restrict__ hi, uint16_t *__restrict__ lo, uint16_t *sh) {
-  const int nt = att_vt_tiles(t_pad);
-  const int head = tile / nt, kv0 = (tile % nt) * ATT_VT_KV;
-  const int th = threadIdx.x, d4 = th & 15;
+// One workgroup per (head, 32-row kv block): its K rows (row-contiguous
+// 32-byte reads, 128-byte runs written) and its v^T fragments (a lane gathers
+// its 8 rows' value, 128-byte runs of a row per load; 1 KB runs written).
+// Rows >= t_kv are zeros.  Bound by its bytes, 8 t n read and 8 t n written:
+// 4.9 us for large-v3's 30.7 MB (7.1 us when v^T went through LDS to row-major
+// planes).
+__global__ __launch_bounds__(256) void k_attn_split(const float *__restrict__ k, int ldk, const float *__restrict__ v,
+                                                    int ldv, int t_kv, int nblk, uint16_t *__restrict__ kv) {
+  const int head = blockIdx.x / nblk, blk = blockIdx.x % nblk, t = threadIdx.x;
+  uint16_t *o = kv + (size_t)blockIdx.x * ATT_BLK;
+  float kx[8], vx[8];
+  const int c = t & 7, n = t >> 3;  // K: row n, values 8 c ..
+  {
+    const int row = blk * ATT_KVB + n;
+    const float4 *src = reinterpret_cast<const float4 *>(k + (size_t)min(row, t_kv - 1) * ldk + head * ATT_DH + 8 * c);
+    const float4 a = src[0], b = src[1];
+    const bool live = row < t_kv;
+    const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int row = (th >> 4) + 16 * u, kv = kv0 + row;
-    float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (kv < t) x = *reinterpret_cast<const float4 *>(v + (size_t)kv * ld + head * ATT_DH + 4 * d4);
-    const int pos = (row & ~15) | attn_vpos(row & 15);
-    const float xs[4] = {x.x, x.y, x.z, x.w};
+    for (int e = 0; e < 8; ++e) kx[e] = live ? x[e] : 0.0f;
+  }
+  const int f = t >> 6, l = t & 63;  // v^T: fragment f, lane l
+  {
+    const float *src = v + head * ATT_DH + (f >> 1) * 32 + (l & 31);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      uint16_t hb, lb;
-      att_split(xs[e], hb, lb);
-      sh[(4 * d4 + e) * ATT_VT_LD + pos] = hb;
-      sh[(ATT_DH + 4 * d4 + e) * ATT_VT_LD + pos] = lb;
+    for (int e = 0; e < 8; ++e) {
+      const int row = blk * ATT_KVB + 16 * (f & 1) + attn_vpos(8 * (l >> 5) + e);
+      const float x = src[(size_t)min(row, t_kv - 1) * ldv];
+      vx[e] = row < t_kv ? x : 0.0f;
     }
   }
-  __syncthreads();
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int c = th + 256 * u;  // (plane, d, 8 positions)
-    const int pl = c >> 9, d = (c >> 3) & 63, ch = c & 7;
-    if (kv0 + 8 * ch < t_pad) {
-      const uint4 w = *reinterpret_cast<const uint4 *>(sh + (pl * ATT_DH + d) * ATT_VT_LD + 8 * ch);
-      *reinterpret_cast<uint4 *>((pl ? lo : hi) + ((size_t)head * ATT_DH + d) * t_pad + kv0 + 8 * ch) = w;
-    }
-  }
-}
-
-// All three splits in one launch: workgroups [0, wq) split q (scaled by
-// 1/8, exact), [wq, wq + wk) split k, the rest split v into v^T
-// (n_head * att_vt_tiles(tkv_pad) workgroups).
-__global__ __launch_bounds__(256) void k_attn_split(const float *__restrict__ q, int ldq, int t_q,
-                                                    const float *__restrict__ k, int ldk, const float *__restrict__ v,
-                                                    int ldv, int t_kv, AttnPlanes P, int n_head, int wq, int wk) {
-  const int bx = blockIdx.x;
-  if (bx < wq) {
-    const size_t idx = (size_t)bx * 256 + threadIdx.x;
-    if (idx < (size_t)n_head * P.tq_pad * 8)
-      att_split_rows(idx, q, ldq, t_q, P.tq_pad, 0.125f, const_cast<uint16_t *>(P.qh), const_cast<uint16_t *>(P.ql));
-  } else if (bx < wq + wk) {
-    const size_t idx = (size_t)(bx - wq) * 256 + threadIdx.x;
-    if (idx < (size_t)n_head * P.tkv_pad * 8)
-      att_split_rows(idx, k, ldk, t_kv, P.tkv_pad, 1.0f, const_cast<uint16_t *>(P.kh), const_cast<uint16_t *>(P.kl));
-  } else {
-    __shared__ __align__(16) uint16_t sh[2 * ATT_DH * ATT_VT_LD];
-    const int tile = bx - wq - wk;
-    if (tile < n_head * att_vt_tiles(P.tkv_pad))  // uniform: the whole workgroup
-      att_split_vt_tile(tile, v, ldv, t_kv, P.tkv_pad, const_cast<uint16_t *>(P.vh), const_cast<uint16_t *>(P.vl),
-                        sh);
-  }
+  const int ko = ((c >> 1) * 64 + 32 * (c & 1) + n) * 8, vo = 2 * ATT_PART + t * 8;
+  att_split8(kx, o + ko, o + ATT_PART + ko);
+  att_split8(vx, o + vo, o + ATT_PART + vo);
 }
 
 // Several decoding states' one-token steps in one self-attention: plane
@@ -197,25 +172,23 @@ struct AttV {
   att_v8h vh[2][2], vl[2][2];
 };
 
-__device__ inline void att_load_k(const AttnPlanes &P, int head, int blk, int h, int n, AttK &o) {
-  const size_t krow = ((size_t)head * P.tkv_pad + (size_t)blk * ATT_KVB + n) * ATT_DH + 8 * h;
+// (base: the block's 4 parts plus this lane's 8 values)
+__device__ inline void att_load_k(const uint16_t *base, AttK &o) {
 #pragma unroll
   for (int s = 0; s < 4; ++s) {
-    o.kh[s] = att_ld(P.kh + krow + 16 * s);
-    o.kl[s] = att_ld(P.kl + krow + 16 * s);
+    o.kh[s] = att_ld(base + s * 512);
+    o.kl[s] = att_ld(base + ATT_PART + s * 512);
   }
 }
 
-__device__ inline void att_load_v(const AttnPlanes &P, int head, int blk, int h, int n, AttV &o) {
+__device__ inline void att_load_v(const uint16_t *base, AttV &o) {
 #pragma unroll
-  for (int dt = 0; dt < 2; ++dt) {
-    const size_t vrow = ((size_t)head * ATT_DH + dt * 32 + n) * P.tkv_pad + (size_t)blk * ATT_KVB + 8 * h;
+  for (int dt = 0; dt < 2; ++dt)
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
-      o.vh[dt][s] = att_ld(P.vh + vrow + 16 * s);
-      o.vl[dt][s] = att_ld(P.vl + vrow + 16 * s);
+      o.vh[dt][s] = att_ld(base + 2 * ATT_PART + (2 * dt + s) * 512);
+      o.vl[dt][s] = att_ld(base + 3 * ATT_PART + (2 * dt + s) * 512);
     }
-  }
 }
 
 // The same K and v^T operands straight from f32 rows (kf, vf with row
@@ -283,25 +256,322 @@ __device__ inline void att_split_v(const AttVRaw &x, AttV &o) {
       }
 }
 
-// Workgroup (blockIdx.x, blockIdx.y) = (ATT_QB query rows from q0, head).
-// Wavefront w takes kv blocks w, w + 2, ...; a causal query row i (at
-// absolute position t_kv - t_q + i) sees kv rows up to its position.
+// The softmax's running state of one query (a lane pair (n, n + 32) holds one):
+// cm, a reference exponent, and lsum, this lane's sum of p = 2^(log2(e) s -
+// cm).  cm is set ATT_PS = 8 below log2(e) times the largest score seen, and
+// moved only when a score passes it by more than ATT_PS + ATT_SLACK (p <= 2^15
+// fits f16): then the output and the sum are rescaled.  Any cm gives the same
+// quotient, so its own rounding cancels; p = 2^8 .. 2^15 at the row's maximum
+// keeps small probabilities' f16 bits (hi + lo hold 2^-24 absolute).  Rescaling
+// at every new maximum moved some query of a tile in nearly every block (a
+// wavefront sees 12 of them at t = 1500).
+constexpr float ATT_PS = 8.0f, ATT_SLACK = 7.0f, ATT_NONE = -1e30f;  // ATT_NONE: no score seen yet
+
+// the largest score of the query's 32 kv rows (s: lane (h, n) holds query n's
+// rows 8 (i / 4) + 4 h + i % 4), as the cm it asks for
+__device__ inline float att_block_max(const att_v16f &s) {
+  float mx = fmaxf(s[0], s[1]);
+#pragma unroll
+  for (int i = 2; i < 16; i += 2) mx = fmaxf(fmaxf(mx, s[i]), s[i + 1]);
+  const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+  return __builtin_fmaf(fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1])), ATT_LOG2E, -ATT_PS);
+}
+// does some query of the wavefront need a new cm?
+__device__ inline bool att_moved(float cm, float cb) { return __builtin_amdgcn_ballot_w64(cb > cm + ATT_SLACK) != 0; }
+__device__ inline void att_rescale(float cb, float &cm, float &lsum, att_v16f (&o)[2]) {
+  const float cnew = cb > cm + ATT_SLACK ? cb : cm;
+  const float alpha = __builtin_amdgcn_exp2f(cm - cnew);
+  lsum *= alpha;
+  o[0] *= alpha;
+  o[1] *= alpha;
+  cm = cnew;
+}
+// p - hi, one mixed-precision FMA each (the compiler converts and subtracts)
+__device__ inline att_v2f att_resid(att_v2f p, att_v2h hi) {
+  att_v2f r;
+  const uint32_t hb = __builtin_bit_cast(uint32_t, hi);
+  asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r.x) : "v"(hb), "v"(p.x));
+  asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r.y) : "v"(hb), "v"(p.y));
+  return r;
+}
+// scores to the P^T operands, one FMA and one exp2 each; their sum to lsum
+__device__ inline void att_probs(const att_v16f &s, float cm, float &lsum, att_v8h (&ph)[2], att_v8h (&pl)[2]) {
+  float s0 = 0.0f, s1 = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 16; i += 2) {
+    const att_v2f p = {__builtin_amdgcn_exp2f(__builtin_fmaf(s[i], ATT_LOG2E, -cm)),
+                       __builtin_amdgcn_exp2f(__builtin_fmaf(s[i + 1], ATT_LOG2E, -cm))};
+    s0 += p.x;
+    s1 += p.y;
+    const att_v2h hi = __builtin_convertvector(p, att_v2h);  // one packed conversion
+    const att_v2f r = att_resid(p, hi);
+    const att_v2h lo = __builtin_convertvector(r, att_v2h);
+    ph[i >> 3][i & 7] = hi.x, ph[i >> 3][(i & 7) + 1] = hi.y;
+    pl[i >> 3][i & 7] = lo.x, pl[i >> 3][(i & 7) + 1] = lo.y;
+  }
+  lsum += s0 + s1;
+}
+
+// the scores of block b that query row q0 + n must not see, to -inf
+__device__ inline void att_mask(att_v16f &s, int b, int h, int t_kv, bool causal, int qpos) {
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int kv = b * ATT_KVB + 8 * (i >> 2) + 4 * h + (i & 3);
+    if (kv >= t_kv || (causal && kv > qpos)) s[i] = -__builtin_huge_valf();
+  }
+}
+
+// XCD-aware order: workgroup id % 8 is its XCD; each XCD takes one contiguous
+// range of (head, query block) in head-major order, so a head's query blocks
+// share their K and v^T operands through one L2
+__device__ inline int att_xcd_order(int id, int total) {
+  const int per = total / 8, rem = total % 8, xcd = id % 8, slot = id / 8;
+  return xcd < rem ? xcd * (per + 1) + slot : rem * (per + 1) + (xcd - rem) * per + slot;
+}
+
+// 8 values of a query row (f32, scaled by 1/8, exact) as hi and lo; rows past
+// the last are zeros
+__device__ inline void att_load_q(const float *__restrict__ qf, int ldq, int row, int t_q, int col, att_v8h &qh,
+                                  att_v8h &ql) {
+  float v[8];
+  if (row < t_q) {
+    const float4 *src = reinterpret_cast<const float4 *>(qf + (size_t)row * ldq + col);
+    const float4 a = src[0], b = src[1];
+    v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = 0.0f;
+  }
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    uint16_t hb, lb;
+    att_split(v[e] * 0.125f, hb, lb);
+    qh[e] = __builtin_bit_cast(_Float16, hb);
+    ql[e] = __builtin_bit_cast(_Float16, lb);
+  }
+}
+
+// Calls of more than 8 query rows.  One workgroup per (32 QT query rows,
+// head); wavefront w of 4 takes kv blocks w, w + 4, ..., its operands straight
+// from the split blocks (K's next block while this one's softmax runs, v^T's
+// at the top of its block), with no barrier until the partial results meet in
+// LDS.  A causal query row i (at absolute position t_kv - t_q + i) sees kv
+// rows up to its position.
+//
+// Bound by the matrix cores' rate under load and the softmax beside it: with
+// loads and softmax taken out, large-v3's layer (20 heads, t = 1500, 35.5
+// GFLOP of f16 products) still takes 31 us, 1.3 PFLOP/s, of 41 us (two
+// wavefronts of 64 queries per row group pair on 960 wavefronts took 53: one
+// wavefront per SIMD, accumulators moving between register files, 16-byte
+// loads).  QT = 2 keeps q's operands in LDS (232 registers, two wavefronts per
+// SIMD) and loads 16 KB per 48 products; QT = 1 loads the same per 24, so it
+// is for calls that 64-row tiles leave short of workgroups: 20 heads 41 against
+// 47 us, but 12 heads 34.4 against 32.9, 6 heads at t = 749 12.7 against 8.5,
+// 227 rows against 1500 (20 heads) 21 against 13 us.  Eight wavefronts per
+// workgroup: 46 (QT = 2) and 57 us (QT = 1).
+//
+// ROWS: K and V come as f32 rows (kf, vf) and are split as they are loaded, for
+// calls of one or two query tiles (no split launch); the operands, and so the
+// results, are the split blocks' bits.
+template <int QT, bool ROWS>
+__global__ __launch_bounds__(64 * ATT_NK, 2) void k_attn_tile(int t_q, int t_kv, int causal, int nqb, int total,
+                                                          const float *__restrict__ qf, int ldq,
+                                                          const uint16_t *__restrict__ kv, int nblk_pad,
+                                                          float *__restrict__ out, int ld_out,
+                                                          const float *__restrict__ kf, int ldk,
+                                                          const float *__restrict__ vf, int ldv) {
+  constexpr int NK = ATT_NK, QB = 32 * QT;
+  constexpr bool QLDS = QT > 1;  // q's operands in LDS (64 registers' worth), else in registers
+  constexpr int XLD = 36;        // floats per row of a 32-value output half in LDS
+  __shared__ __align__(16) float xo[NK * QB * XLD];  // q's operands, then the partial outputs
+  __shared__ float xm[NK][QB], xl[NK][QB], xinv[QB];
+  static_assert(sizeof(xo) >= (size_t)QT * 8 * 1024, "q's operands");
+  const int l = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int h = l >> 5, n = l & 31;
+  const int lin = att_xcd_order(blockIdx.x, total);
+  const int head = lin / nqb, q0 = (lin % nqb) * QB;
+  const int off = t_kv - t_q;  // absolute position of query row 0
+  const int kv_end = causal ? min(t_kv, off + q0 + QB) : t_kv;
+  const int nblk = (kv_end + ATT_KVB - 1) / ATT_KVB;
+  const uint16_t *base = kv + (size_t)head * nblk_pad * ATT_BLK + l * 8;
+
+  AttK kk;
+  AttV vv;
+  AttKRaw kr;
+  AttVRaw vr;
+  auto load_k = [&](int blk) __attribute__((always_inline)) {
+    if constexpr (ROWS) att_load_k_raw(kf, ldk, t_kv, head, blk, h, n, kr);
+    else att_load_k(base + (size_t)blk * ATT_BLK, kk);
+  };
+  auto load_v = [&](int blk) __attribute__((always_inline)) {
+    if constexpr (ROWS) att_load_v_raw(vf, ldv, t_kv, head, blk, h, n, vr);
+    else att_load_v(base + (size_t)blk * ATT_BLK, vv);
+  };
+  if (wv < nblk) load_k(wv);
+
+  // q's operands: fragment (qt, s), hi then lo
+  att_v8h qh[QLDS ? 1 : 4], ql[QLDS ? 1 : 4];
+  uint16_t *qs = reinterpret_cast<uint16_t *>(xo) + l * 8;
+  if constexpr (QLDS) {
+#pragma unroll
+    for (int f = wv; f < 4 * QT; f += NK) {
+      att_v8h a, b;
+      att_load_q(qf, ldq, q0 + (f >> 2) * 32 + n, t_q, head * ATT_DH + 8 * h + 16 * (f & 3), a, b);
+      *reinterpret_cast<uint4 *>(qs + 2 * f * 512) = __builtin_bit_cast(uint4, a);
+      *reinterpret_cast<uint4 *>(qs + (2 * f + 1) * 512) = __builtin_bit_cast(uint4, b);
+    }
+    __syncthreads();
+  } else {
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+      att_load_q(qf, ldq, q0 + n, t_q, head * ATT_DH + 8 * h + 16 * s, qh[s], ql[s]);
+  }
+
+  att_v16f o[QT][2];  // O^T
+  float cm[QT], lsum[QT];
+#pragma unroll
+  for (int qt = 0; qt < QT; ++qt) {
+    o[qt][0] = (att_v16f){};
+    o[qt][1] = (att_v16f){};
+    cm[qt] = ATT_NONE;
+    lsum[qt] = 0.0f;
+  }
+  int b = wv;
+  att_v16f s[QT];
+  float cb[QT];
+  // block b's scores and maxima, K's next block requested behind them
+  auto scores = [&]() __attribute__((always_inline)) {
+    // (an offset the compiler cannot see through: it would keep all of q's
+    // operands in registers across the loop, and spill)
+    int qo = l * 8;
+    if constexpr (QLDS) asm volatile("" : "+v"(qo));
+    if constexpr (ROWS) att_split_k(kr, b * ATT_KVB + n < t_kv, kk);
+    const uint16_t *qp = reinterpret_cast<const uint16_t *>(xo) + qo;
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) {
+      s[qt] = (att_v16f){};
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        if constexpr (QLDS)
+          att_mma3(kk.kh[k], kk.kl[k], att_ld(qp + 2 * (4 * qt + k) * 512), att_ld(qp + (2 * (4 * qt + k) + 1) * 512),
+                   s[qt]);
+        else
+          att_mma3(kk.kh[k], kk.kl[k], qh[k], ql[k], s[qt]);
+      }
+    }
+    load_k(min(b + NK, nblk - 1));
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) {
+      const int tq0 = q0 + qt * 32;
+      if ((b + 1) * ATT_KVB > t_kv || (causal && (b + 1) * ATT_KVB - 1 > off + tq0))
+        att_mask(s[qt], b, h, t_kv, causal, off + tq0 + n);
+      cb[qt] = att_block_max(s[qt]);
+    }
+  };
+  // Two loops, so that the common path has no rescale to merge with: beside
+  // one the compiler copied all of O^T in every block (50 against 47 us with
+  // QT = 1 at 20 heads)
+  if (b < nblk) {
+    load_v(b);
+    scores();
+    for (;;) {
+#pragma unroll
+      for (int qt = 0; qt < QT; ++qt) att_rescale(cb[qt], cm[qt], lsum[qt], o[qt]);
+      bool moved;
+      do {
+        if constexpr (ROWS) att_split_v(vr, vv);
+#pragma unroll
+        for (int qt = 0; qt < QT; ++qt) {
+          att_v8h ph[2], pl[2];
+          att_probs(s[qt], cm[qt], lsum[qt], ph, pl);
+#pragma unroll
+          for (int k = 0; k < 2; ++k)
+#pragma unroll
+            for (int dt = 0; dt < 2; ++dt) att_mma3(vv.vh[dt][k], vv.vl[dt][k], ph[k], pl[k], o[qt][dt]);
+        }
+        b += NK;
+        if (b >= nblk) break;
+        load_v(b);
+        scores();
+        moved = false;
+#pragma unroll
+        for (int qt = 0; qt < QT; ++qt) moved = moved || att_moved(cm[qt], cb[qt]);
+      } while (!moved);
+      if (b >= nblk) break;
+    }
+  }
+
+  // the NK partial states meet: every wavefront's output scaled to the common
+  // maximum, summed in wavefront order, divided by the common sum
+#pragma unroll
+  for (int qt = 0; qt < QT; ++qt) {
+    const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(lsum[qt]), __float_as_uint(lsum[qt]), false, false);
+    const float lt = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
+    if (h == 0) {
+      xm[wv][qt * 32 + n] = cm[qt];
+      xl[wv][qt * 32 + n] = lt;
+    }
+  }
+  __syncthreads();  // every wavefront is done with q's operands too
+#pragma unroll
+  for (int qt = 0; qt < QT; ++qt) {
+    float mu = ATT_NONE;
+#pragma unroll
+    for (int w = 0; w < NK; ++w) mu = fmaxf(mu, xm[w][qt * 32 + n]);
+    if (wv == 0 && h == 0) {
+      float den = 0.0f;
+#pragma unroll
+      for (int w = 0; w < NK; ++w) den += xl[w][qt * 32 + n] * __builtin_amdgcn_exp2f(xm[w][qt * 32 + n] - mu);
+      xinv[qt * 32 + n] = 1.0f / den;
+    }
+    const float sc = __builtin_amdgcn_exp2f(cm[qt] - mu);
+    o[qt][0] *= sc;
+    o[qt][1] *= sc;
+  }
+#pragma unroll
+  for (int dt = 0; dt < 2; ++dt) {
+    if (dt) __syncthreads();  // the first half has been read
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<float4 *>(&xo[((wv * QT + qt) * 32 + n) * XLD + 8 * g + 4 * h]) =
+            make_float4(o[qt][dt][4 * g], o[qt][dt][4 * g + 1], o[qt][dt][4 * g + 2], o[qt][dt][4 * g + 3]);
+    __syncthreads();
+#pragma unroll
+    for (int c = threadIdx.x; c < QB * 8; c += 64 * NK) {
+      const int row = c >> 3, c4 = c & 7;
+      float4 y = *reinterpret_cast<const float4 *>(&xo[row * XLD + 4 * c4]);
+#pragma unroll
+      for (int w = 1; w < NK; ++w) {
+        const float4 x = *reinterpret_cast<const float4 *>(&xo[(w * QB + row) * XLD + 4 * c4]);
+        y.x += x.x, y.y += x.y, y.z += x.z, y.w += x.w;
+      }
+      const float inv = xinv[row];
+      if (q0 + row < t_q)
+        *reinterpret_cast<float4 *>(out + (size_t)(q0 + row) * ld_out + head * ATT_DH + dt * 32 + 4 * c4) =
+            make_float4(y.x * inv, y.y * inv, y.z * inv, y.w * inv);
+    }
+  }
+}
+
+// Calls of at most 8 query rows.  Workgroup (blockIdx.x, blockIdx.y) = (32
+// query rows, head); wavefront w takes kv
+// blocks w, w + 2, ...; a causal query row i (at absolute position t_kv - t_q
+// + i) sees kv rows up to its position.
 //
 // Split kv (few query blocks, e.g. one decoding step): with part != NULL,
 // workgroup z of gridDim.z takes the z-th run of the kv blocks and writes
-// its unnormalized O (2^12-scaled), running maximum and sum to part;
-// k_attn_combine merges the runs.
+// its unnormalized O (2^12-scaled), running maximum and sum to
+// part; k_attn_combine merges the runs.
 //
-// With qf != NULL the queries come as f32 rows (qf, ldq) and are scaled and
-// split here, exactly as k_attn_split would store them (P.qh, P.ql unused):
-// the decoder's cross-attention, whose K and v^T planes are kept, then needs
-// no split launch.  QT: 32-query tiles per workgroup (2, or 1 for calls of at
-// most 32 query rows: a decoding step then does half the products and
-// softmax work; a query row's arithmetic does not depend on QT).
-// ROWS: K and V come as f32 rows too (kf, vf) and are split
-// here as well (the P planes are unused): calls of one query block (a
-// decoding step's self-attention over its cache) then need no split launch;
-// the operands are the planes' values, so the results are the same bits.
+// The queries come as f32 rows and are scaled and split here; K and v^T as
+// split blocks (P: the decoder's cross-attention keeps them).
+// ROWS: K and V come as f32 rows too (kf, vf) and are split here as well (P's
+// blocks are unused): a decoding step's self-attention over its cache then
+// needs no split launch; the operands are the blocks' values, so the results
+// are the same bits.
 // The scalars and row pointers lead the arguments: the first 14 dwords
 // arrive in SGPRs when the waves start (kernarg preloading), so a decoding
 // step's attention requests its rows without first reading the argument
@@ -319,33 +589,22 @@ __device__ void attn_block_records(uint8_t *rec, int i, int bl, int lt, int mr, 
 // stored into the caches at that row (by the kv split's first run).
 // rec (BEAMS, no kv split): also the output rows' activation records for
 // the next product.  rec_hd = heads per beam | offset term << 8 | beams << 16.
-template <bool ROWS, int QT, bool BEAMS = false>
+template <bool ROWS, bool BEAMS = false>
 __global__ __launch_bounds__(128) void k_attn(int t_q, int t_kv, int gw, int nx, const float *__restrict__ qf,
                                               int ldq, const float *__restrict__ kf, int ldk,
                                               const float *__restrict__ vf, int ldv, float *__restrict__ out,
                                               int ld_out, float *__restrict__ part, AttnPlanes P,
                                               uint8_t *__restrict__ rec, int rec_hd, BeamCaches C) {
   const int causal = gw & 1, gz = (gw >> 1) & 127, gy = gw >> 8;
-  constexpr int QB = 32 * QT;  // query rows per workgroup
-  constexpr float LOG2E = 1.4426950408889634f;
+  constexpr int QB = 32;  // query rows per workgroup
   constexpr float NEG_INF = -__builtin_huge_valf();
   __shared__ __align__(16) float xo[QB * (ATT_DH + 4)];  // partial O^T exchange, then the output tile
-  __shared__ float xm[QT * 64], xl[QT * 64];
+  __shared__ float xm[64], xl[64];
   const int l = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int h = l >> 5, n = l & 31;
-  // XCD-aware order: workgroup id % 8 is its XCD; each XCD takes one
-  // contiguous range of (head, query block) in head-major order, so a
-  // head's query blocks share their K and v^T planes through one L2
-  int head, q0;
-  {
-    const int nqb = nx, total = nqb * gy;
-    const int id = blockIdx.y * nqb + blockIdx.x;
-    const int per = total / 8, rem = total % 8, xcd = id % 8, slot = id / 8;
-    const int lin = xcd < rem ? xcd * (per + 1) + slot : rem * (per + 1) + (xcd - rem) * per + slot;
-    head = lin / nqb;
-    q0 = (lin % nqb) * QB;
-  }
+  const int lin = att_xcd_order(blockIdx.y * nx + blockIdx.x, nx * gy);
+  const int head = lin / nx, q0 = (lin % nx) * QB;
   const int off = t_kv - t_q;  // absolute position of query row 0
   const int kv_end = causal ? min(t_kv, off + q0 + QB) : t_kv;
   const int nblk_all = (kv_end + ATT_KVB - 1) / ATT_KVB;
@@ -353,45 +612,11 @@ __global__ __launch_bounds__(128) void k_attn(int t_q, int t_kv, int gw, int nx,
   const int b_begin = min(nblk_all, (int)blockIdx.z * cs);
   const int nblk = min(nblk_all, b_begin + cs);               // this workgroup: blocks [b_begin, nblk)
 
-  att_v8h qh[QT][4], ql[QT][4];
+  att_v8h qh[4], ql[4];
 #pragma unroll
-  for (int qt = 0; qt < QT; ++qt) {
-    const size_t qrow = ((size_t)head * P.tq_pad + q0 + qt * 32 + n) * ATT_DH + 8 * h;
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      if (qf) {
-        const int row = q0 + qt * 32 + n;
-        float v[8];
-        if (row < t_q) {
-          const float4 *src = reinterpret_cast<const float4 *>(qf + (size_t)row * ldq + head * ATT_DH + 8 * h + 16 * s);
-          const float4 a = src[0], b = src[1];
-          v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
-        } else {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) v[e] = 0.0f;
-        }
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          uint16_t hb, lb;
-          att_split(v[e] * 0.125f, hb, lb);
-          qh[qt][s][e] = __builtin_bit_cast(_Float16, hb);
-          ql[qt][s][e] = __builtin_bit_cast(_Float16, lb);
-        }
-      } else {
-        qh[qt][s] = att_ld(P.qh + qrow + 16 * s);
-        ql[qt][s] = att_ld(P.ql + qrow + 16 * s);
-      }
-    }
-  }
-  att_v16f o[QT][2];  // O^T
-  float m[QT], lsum[QT];
-#pragma unroll
-  for (int qt = 0; qt < QT; ++qt) {
-    o[qt][0] = (att_v16f){};
-    o[qt][1] = (att_v16f){};
-    m[qt] = NEG_INF;
-    lsum[qt] = 0.0f;
-  }
+  for (int s = 0; s < 4; ++s) att_load_q(qf, ldq, q0 + n, t_q, head * ATT_DH + 8 * h + 16 * s, qh[s], ql[s]);
+  att_v16f o[2] = {(att_v16f){}, (att_v16f){}};  // O^T
+  float m = NEG_INF, lsum = 0.0f;
 
   // K one block ahead; V is loaded at the top of its block and first used
   // after the scores and the softmax
@@ -401,6 +626,7 @@ __global__ __launch_bounds__(128) void k_attn(int t_q, int t_kv, int gw, int nx,
   AttVRaw vr;
   // this plane's K and V rows (BEAMS: its beam's caches and new row)
   const float *kfp = kf, *vfp = vf, *klast = nullptr, *vlast = nullptr;
+  const uint16_t *base = P.kv + (size_t)head * (P.tkv_pad / ATT_KVB) * ATT_BLK + l * 8;
   int hkv = head;
   if constexpr (BEAMS) {
     const int hpb = rec_hd & 255, bb = head / hpb;
@@ -417,7 +643,7 @@ __global__ __launch_bounds__(128) void k_attn(int t_q, int t_kv, int gw, int nx,
   }
   if (b_begin + wv < nblk) {
     if constexpr (ROWS) att_load_k_raw(kfp, ldk, t_kv, hkv, b_begin + wv, h, n, kr_cur, klast);
-    else att_load_k(P, head, b_begin + wv, h, n, cur);
+    else att_load_k(base + (size_t)(b_begin + wv) * ATT_BLK, cur);
   }
   for (int b = b_begin + wv; b < nblk; b += 2) {
     if constexpr (ROWS) {
@@ -425,67 +651,47 @@ __global__ __launch_bounds__(128) void k_attn(int t_q, int t_kv, int gw, int nx,
       if (b + 2 < nblk) att_load_k_raw(kfp, ldk, t_kv, hkv, b + 2, h, n, kr_nxt, klast);
       att_split_k(kr_cur, b * ATT_KVB + n < t_kv, cur);
     } else {
-      att_load_v(P, head, b, h, n, vb);
-      if (b + 2 < nblk) att_load_k(P, head, b + 2, h, n, nxt);
+      att_load_v(base + (size_t)b * ATT_BLK, vb);
+      if (b + 2 < nblk) att_load_k(base + (size_t)(b + 2) * ATT_BLK, nxt);
     }
-    // both query tiles' scores first, so the softmax of one tile can run on
-    // the VALU while the matrix cores work on the other
-    att_v16f s[QT];
+    att_v16f s = (att_v16f){};
 #pragma unroll
-    for (int qt = 0; qt < QT; ++qt) {
-      s[qt] = (att_v16f){};
-#pragma unroll
-      for (int k = 0; k < 4; ++k) att_mma3(cur.kh[k], cur.kl[k], qh[qt][k], ql[qt][k], s[qt]);
-    }
+    for (int k = 0; k < 4; ++k) att_mma3(cur.kh[k], cur.kl[k], qh[k], ql[k], s);
     if constexpr (ROWS) att_split_v(vr, vb);
+    if ((b + 1) * ATT_KVB > t_kv || (causal && (b + 1) * ATT_KVB - 1 > off + q0))
+      att_mask(s, b, h, t_kv, causal, off + q0 + n);
+    att_v8h ph[2], pl[2];
+    float mx = s[0];
 #pragma unroll
-    for (int qt = 0; qt < QT; ++qt) {
-      // lane (h, n): s[qt][i] = score of query q0 + 32 qt + n against kv
-      // row 32 b + 8 (i / 4) + 4 h + i % 4
-      const int tq0 = q0 + qt * 32;
-      const bool partial = (b + 1) * ATT_KVB > t_kv || (causal && (b + 1) * ATT_KVB - 1 > off + tq0);
-      if (partial) {
-        const int qpos = off + tq0 + n;
+    for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[i]);
+    mx = fmaxf(mx, __shfl_xor(mx, 32));
+    const float mnew = fmaxf(m, mx);
+    const float mu = mnew == NEG_INF ? 0.0f : mnew;  // a query with nothing visible yet
+    float ps = 0.0f;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const int kv = b * ATT_KVB + 8 * (i >> 2) + 4 * h + (i & 3);
-          if (kv >= t_kv || (causal && kv > qpos)) s[qt][i] = NEG_INF;
-        }
-      }
-      float mx = s[qt][0];
-#pragma unroll
-      for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[qt][i]);
-      mx = fmaxf(mx, __shfl_xor(mx, 32));
-      const float mnew = fmaxf(m[qt], mx);
-      const float mu = mnew == NEG_INF ? 0.0f : mnew;  // a column with nothing visible yet
-      float ps = 0.0f;
-      att_v8h ph[2], pl[2];
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const float p = __builtin_amdgcn_exp2f((s[qt][i] - mu) * LOG2E);
-        ps += p;
-        // P enters the products as 2^12 p, so that small probabilities keep
-        // their f16 bits; the output is divided by 2^12 lsum at the end
-        const float p12 = p * ATT_PS;
-        const _Float16 ph1 = (_Float16)p12;
-        ph[i >> 3][i & 7] = ph1;
-        pl[i >> 3][i & 7] = (_Float16)(p12 - (float)ph1);
-      }
-      // rescale only when some column's maximum moved (rare after the
-      // first blocks)
-      if (__builtin_amdgcn_ballot_w64(mnew != m[qt])) {
-        const float alpha = __builtin_amdgcn_exp2f((m[qt] - mu) * LOG2E);
-        lsum[qt] *= alpha;
-#pragma unroll
-        for (int dt = 0; dt < 2; ++dt) o[qt][dt] *= alpha;
-      }
-      m[qt] = mnew;
-      lsum[qt] += ps;
-#pragma unroll
-      for (int dt = 0; dt < 2; ++dt)
-#pragma unroll
-        for (int k = 0; k < 2; ++k) att_mma3(vb.vh[dt][k], vb.vl[dt][k], ph[k], pl[k], o[qt][dt]);
+    for (int i = 0; i < 16; ++i) {
+      const float p = __builtin_amdgcn_exp2f((s[i] - mu) * ATT_LOG2E);
+      ps += p;
+      // P enters the products as 2^12 p, so that small probabilities keep
+      // their f16 bits; the output is divided by 2^12 lsum at the end
+      const float p12 = p * ATT_STEP_PS;
+      const _Float16 ph1 = (_Float16)p12;
+      ph[i >> 3][i & 7] = ph1;
+      pl[i >> 3][i & 7] = (_Float16)(p12 - (float)ph1);
     }
+    // rescale only when some query's maximum moved
+    if (__builtin_amdgcn_ballot_w64(mnew != m)) {
+      const float alpha = __builtin_amdgcn_exp2f((m - mu) * ATT_LOG2E);
+      lsum *= alpha;
+      o[0] *= alpha;
+      o[1] *= alpha;
+    }
+    m = mnew;
+    lsum += ps;
+#pragma unroll
+    for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+      for (int k = 0; k < 2; ++k) att_mma3(vb.vh[dt][k], vb.vl[dt][k], ph[k], pl[k], o[dt]);
     if constexpr (ROWS) kr_cur = kr_nxt;
     else cur = nxt;
   }
@@ -493,51 +699,42 @@ __global__ __launch_bounds__(128) void k_attn(int t_q, int t_kv, int gw, int nx,
   // wavefront 1 hands its partial state to wavefront 0
   if (wv == 1) {
 #pragma unroll
-    for (int qt = 0; qt < QT; ++qt) {
+    for (int dt = 0; dt < 2; ++dt)
 #pragma unroll
-      for (int dt = 0; dt < 2; ++dt)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) xo[((qt * 2 + dt) * 16 + i) * 64 + l] = o[qt][dt][i];
-      xm[qt * 64 + l] = m[qt];
-      xl[qt * 64 + l] = lsum[qt];
-    }
+      for (int i = 0; i < 16; ++i) xo[(dt * 16 + i) * 64 + l] = o[dt][i];
+    xm[l] = m;
+    xl[l] = lsum;
   }
   __syncthreads();
   if (wv == 0) {
-#pragma unroll
-    for (int qt = 0; qt < QT; ++qt) {
-      const float m1 = xm[qt * 64 + l], l1 = xl[qt * 64 + l];
-      const float mm = fmaxf(m[qt], m1);
-      const float mu = mm == NEG_INF ? 0.0f : mm;
-      const float s0 = __builtin_amdgcn_exp2f((m[qt] - mu) * LOG2E), s1 = __builtin_amdgcn_exp2f((m1 - mu) * LOG2E);
-      float lt = lsum[qt] * s0 + l1 * s1;
-      lt += __shfl_xor(lt, 32);
-      const float inv = part ? 1.0f : 1.0f / (lt * ATT_PS);
-      if (part && h == 0 && q0 + qt * 32 + n < t_q) {
-        const size_t pr = ((size_t)blockIdx.z * gy + head) * P.tq_pad + q0 + qt * 32 + n;
-        float *pml = part + (size_t)gz * gy * P.tq_pad * ATT_DH;
-        pml[2 * pr] = mm;
-        pml[2 * pr + 1] = lt;
-      }
-#pragma unroll
-      for (int dt = 0; dt < 2; ++dt)
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-          o[qt][dt][i] = (o[qt][dt][i] * s0 + xo[((qt * 2 + dt) * 16 + i) * 64 + l] * s1) * inv;
+    const float m1 = xm[l], l1 = xl[l];
+    const float mm = fmaxf(m, m1);
+    const float mu = mm == NEG_INF ? 0.0f : mm;
+    const float s0 = __builtin_amdgcn_exp2f((m - mu) * ATT_LOG2E), s1 = __builtin_amdgcn_exp2f((m1 - mu) * ATT_LOG2E);
+    float lt = lsum * s0 + l1 * s1;
+    lt += __shfl_xor(lt, 32);
+    const float inv = part ? 1.0f : 1.0f / (lt * ATT_STEP_PS);
+    if (part && h == 0 && q0 + n < t_q) {
+      const size_t pr = ((size_t)blockIdx.z * gy + head) * P.tq_pad + q0 + n;
+      float *pml = part + (size_t)gz * gy * P.tq_pad * ATT_DH;
+      pml[2 * pr] = mm;
+      pml[2 * pr + 1] = lt;
     }
+#pragma unroll
+    for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) o[dt][i] = (o[dt][i] * s0 + xo[(dt * 16 + i) * 64 + l] * s1) * inv;
   }
   __syncthreads();
-  // the output tile [64 queries][64 d] through LDS, then row-contiguous stores
+  // the output tile [32 queries][64 d] through LDS, then row-contiguous stores
   constexpr int LD = ATT_DH + 4;
   if (wv == 0) {
 #pragma unroll
-    for (int qt = 0; qt < QT; ++qt)
+    for (int dt = 0; dt < 2; ++dt)
 #pragma unroll
-      for (int dt = 0; dt < 2; ++dt)
-#pragma unroll
-        for (int g = 0; g < 4; ++g)
-          *reinterpret_cast<float4 *>(&xo[(qt * 32 + n) * LD + dt * 32 + 8 * g + 4 * h]) =
-              make_float4(o[qt][dt][4 * g], o[qt][dt][4 * g + 1], o[qt][dt][4 * g + 2], o[qt][dt][4 * g + 3]);
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<float4 *>(&xo[n * LD + dt * 32 + 8 * g + 4 * h]) =
+            make_float4(o[dt][4 * g], o[dt][4 * g + 1], o[dt][4 * g + 2], o[dt][4 * g + 3]);
   }
   __syncthreads();
 #pragma unroll
@@ -560,8 +757,8 @@ __global__ __launch_bounds__(128) void k_attn(int t_q, int t_kv, int gw, int nx,
   }
 }
 
-// Merge nsplit runs of k_attn: out = sum_z O_z 2^(m_z - m) / (2^12 sum_z l_z
-// 2^(m_z - m)), m the largest run maximum (runs that saw nothing have
+// Merge nsplit runs of k_attn: out = sum_z O_z e^(m_z - m) / (2^12 sum_z l_z
+// e^(m_z - m)), m the largest run maximum (runs that saw nothing have
 // m = -inf and weigh 0).  One thread per (query, head, d).
 // (defined with the decode GEMV: one query row's block of the output as the
 // next product's activation record)
@@ -573,7 +770,6 @@ __device__ void combine_records(uint8_t *rec, int row, int col, int mr, float x,
 __global__ __launch_bounds__(256) void k_attn_combine(const float *__restrict__ part, int nsplit, int n_head,
                                                       int tq_pad, int t_q, float *__restrict__ out, int ld_out,
                                                       uint8_t *__restrict__ rec, int rec_off) {
-  constexpr float LOG2E = 1.4426950408889634f;
   constexpr float NEG_INF = -__builtin_huge_valf();
   const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
   if (idx >= (size_t)t_q * n_head * ATT_DH) return;
@@ -600,13 +796,13 @@ __global__ __launch_bounds__(256) void k_attn_combine(const float *__restrict__ 
   float num = 0.0f, den = 0.0f;
 #pragma unroll
   for (int z = 0; z < ATT_MAX_SPLIT; ++z) {
-    const float w = __builtin_amdgcn_exp2f((mz[z] - mu) * LOG2E);
+    const float w = __builtin_amdgcn_exp2f((mz[z] - mu) * ATT_LOG2E);
     if (z < nsplit && w > 0.0f) {  // a run that saw no key holds no output
       num += oz[z] * w;
       den += lz[z] * w;
     }
   }
-  const float y = num / (den * ATT_PS);
+  const float y = num / (den * ATT_STEP_PS);
   out[(size_t)q * ld_out + head * ATT_DH + d] = y;
   if (rec) combine_records(rec, q, head * ATT_DH + d, t_q, y, rec_off);  // whole wavefronts (uniform)
 }

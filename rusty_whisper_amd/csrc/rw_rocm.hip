@@ -994,7 +994,7 @@ static int check_matmul_args(const rw_weight *w, const void *a, size_t m, size_t
 // Workspace of one attention call: the f16 pairs of q, k and v^T.
 struct AttnLayout {
   int n_head, tq_pad, tkv_pad, nsplit;
-  size_t off_qh, off_ql, off_kh, off_kl, off_vh, off_vl, off_part, bytes;
+  size_t off_kv, off_part, bytes;
 };
 
 // few (query block, head) workgroups -- a decoding step: split the kv
@@ -1019,16 +1019,12 @@ static AttnLayout attn_layout(size_t t_q, size_t t_kv, size_t n_state, bool kv_p
   L.n_head = (int)(n_state / ATT_DH);
   L.tq_pad = (int)align_up(t_q, ATT_QB);
   L.tkv_pad = (int)align_up(t_kv, ATT_KVB);
-  const size_t qb = (size_t)L.n_head * L.tq_pad * ATT_DH * 2;
-  const size_t kb = kv_planes ? (size_t)L.n_head * L.tkv_pad * ATT_DH * 2 : 0;
-  L.off_qh = 0;
-  L.off_ql = align_up(L.off_qh + qb, 256);
-  L.off_kh = align_up(L.off_ql + qb, 256);
-  L.off_kl = align_up(L.off_kh + kb, 256);
-  L.off_vh = align_up(L.off_kl + kb, 256);
-  L.off_vl = align_up(L.off_vh + kb, 256);
+  // (the size still counts room for q's pairs, as callers were told; q is
+  // split in registers)
+  L.off_kv = align_up(2 * (size_t)L.n_head * L.tq_pad * ATT_DH * 2, 256);
+  const size_t kv = kv_planes ? (size_t)L.n_head * (L.tkv_pad / ATT_KVB) * ATT_BLK * 2 : 0;
   L.nsplit = attn_nsplit((size_t)(L.tq_pad / ATT_QB) * L.n_head, cdiv(t_kv, ATT_KVB));
-  L.off_part = align_up(L.off_vl + kb, 256);
+  L.off_part = align_up(L.off_kv + kv, 256);
   const size_t part = L.nsplit > 1 ? (size_t)L.nsplit * L.n_head * L.tq_pad * (ATT_DH + 2) * 4 : 0;
   L.bytes = align_up(L.off_part + part, 256);
   return L;
@@ -1056,6 +1052,15 @@ static int check_attn_args(const float *q, size_t ldq, const float *k, size_t ld
   return RW_OK;
 }
 
+// K and v^T rows of every head -> the operand blocks of k_attn_tile / k_attn
+static int launch_attn_split(const float *k, size_t ldk, const float *v, size_t ldv, size_t t_kv, int n_head,
+                             uint16_t *kv, int nblk, hipStream_t s) {
+  hipLaunchKernelGGL(k_attn_split, dim3((unsigned)(n_head * nblk)), dim3(256), 0, s, k, (int)ldk, v, (int)ldv,
+                     (int)t_kv, nblk, kv);
+  LAUNCH_TRY("k_attn_split");
+  return RW_OK;
+}
+
 // rec (2-8 query rows): where the kv is split, the merge also writes the
 // output rows' activation records for the next product (offset term
 // rec_off), and *rec_done says whether it did.
@@ -1065,9 +1070,6 @@ static int run_attention(const float *q, size_t ldq, const float *k, size_t ldk,
                          int rec_off = 0, bool *rec_done = nullptr) {
   if (rec_done) *rec_done = false;
   char *b = (char *)ws;
-  uint16_t *qh = (uint16_t *)(b + L.off_qh), *ql = (uint16_t *)(b + L.off_ql);
-  uint16_t *kh = (uint16_t *)(b + L.off_kh), *kl = (uint16_t *)(b + L.off_kl);
-  uint16_t *vh = (uint16_t *)(b + L.off_vh), *vl = (uint16_t *)(b + L.off_vl);
   if (t_kv == 0) {  // no keys: every output row is the empty sum
     const size_t nz = t_q * (size_t)n_head * ATT_DH;
     hipLaunchKernelGGL(k_attn_zero, dim3((unsigned)cdiv(nz, 256)), dim3(256), 0, s, out, (int)ldo, (int)t_q,
@@ -1075,47 +1077,44 @@ static int run_attention(const float *q, size_t ldq, const float *k, size_t ldk,
     LAUNCH_TRY("k_attn_zero");
     return RW_OK;
   }
-  // k_attn splits q (f32, scaled by 1/8) as it loads it; K and v^T are split
-  // here, or were split before (kv_split: the decoder's cross-attention)
-  // planes padded to this call's t_kv (the layout may be sized for a longer
-  // one, e.g. a decoder's n_ctx)
-  AttnPlanes P{qh, ql, kh, kl, vh, vl, L.tq_pad, (int)std::min<size_t>(align_up(t_kv, ATT_KVB), L.tkv_pad)};
-  if (kv_split) {
-    P.kh = kv_split->kh, P.kl = kv_split->kl, P.vh = kv_split->vh, P.vl = kv_split->vl;
-    P.tkv_pad = kv_split->tkv_pad;
-  }
-  // one query block against k and v rows (a decoding step's self-attention):
-  // k_attn splits q, K and V as it loads them
-  const bool rows = !kv_split && L.tq_pad == ATT_QB;
-  if (!kv_split && !rows) {  // k and v only: k_attn splits q as it loads it
-    const size_t nk = (size_t)n_head * P.tkv_pad * 8;
-    const int wk = (int)cdiv(nk, 256);
-    const int wv = n_head * (int)cdiv(P.tkv_pad, ATT_VT_KV);  // v^T: one workgroup per (head, 64 positions)
-    hipLaunchKernelGGL(k_attn_split, dim3((unsigned)(wk + wv)), dim3(256), 0, s, q, (int)ldq, (int)t_q, k,
-                       (int)ldk, v, (int)ldv, (int)t_kv, P, n_head, 0, wk);
-    LAUNCH_TRY("k_attn_split");
+  // the kernels split q (f32, scaled by 1/8) as they load it; K and v^T were
+  // split before (kv_split: the decoder's cross-attention), are split here
+  // into blocks padded to this call's t_kv (the layout may be sized for a
+  // longer one, e.g. a decoder's n_ctx), or, for at most 64 query rows (each
+  // of at most two tiles splits them again), as the kernel loads them
+  AttnPlanes P{(uint16_t *)(b + L.off_kv), L.tq_pad, (int)std::min<size_t>(align_up(t_kv, ATT_KVB), L.tkv_pad)};
+  if (kv_split) P.kv = kv_split->kv, P.tkv_pad = kv_split->tkv_pad;
+  const int nblk = P.tkv_pad / ATT_KVB;
+  const bool rows = !kv_split && t_q <= (size_t)ATT_ROWS_MAX;
+  if (t_q > (size_t)ATT_STEP_MAX) {
+    if (!kv_split && !rows)
+      RW_TRY(launch_attn_split(k, ldk, v, ldv, t_kv, n_head, (uint16_t *)(b + L.off_kv), nblk, s));
+    // 64 query rows per workgroup where those fill 3/4 of the 512 workgroup
+    // places (two per CU), else 32 (k_attn_tile has both sides measured)
+    const bool two = !rows && cdiv(t_q, 64) * (size_t)n_head >= 384;
+    const int nqb = (int)cdiv(t_q, two ? 64 : 32), total = nqb * n_head;
+#define RW_ATT_TILE(QT, ROWS)                                                                                      \
+  hipLaunchKernelGGL((k_attn_tile<QT, ROWS>), dim3((unsigned)total), dim3(64 * ATT_NK), 0, s, (int)t_q, (int)t_kv, \
+                     causal, nqb, total, q, (int)ldq, P.kv, nblk, out, (int)ldo, k, (int)ldk, v, (int)ldv)
+    if (rows) RW_ATT_TILE(1, true);
+    else if (two) RW_ATT_TILE(2, false);
+    else RW_ATT_TILE(1, false);
+#undef RW_ATT_TILE
+    LAUNCH_TRY("k_attn_tile");
+    return RW_OK;
   }
   // this call's split (the layout's is for its longest kv; the rule grows
   // with the kv length, so this one fits the layout's part buffer)
-  const int nsplit = std::min(L.nsplit, attn_nsplit((size_t)(L.tq_pad / ATT_QB) * n_head, cdiv(t_kv, ATT_KVB)));
+  const int nsplit = std::min(L.nsplit, attn_nsplit((size_t)n_head, cdiv(t_kv, ATT_KVB)));
   float *part = nsplit > 1 ? (float *)(b + L.off_part) : nullptr;
-  // calls of at most 32 query rows run one 32-query tile per workgroup
-  const bool one_tile = t_q <= 32;
-  const dim3 grid(one_tile ? 1u : (unsigned)(L.tq_pad / ATT_QB), (unsigned)n_head, (unsigned)nsplit);
-  const int cz = causal ? 1 : 0;
-  const int gw = cz | nsplit << 1 | n_head << 8;  // k_attn's packed grid
-  if (rows && one_tile)
-    hipLaunchKernelGGL((k_attn<true, 1>), grid, dim3(128), 0, s, (int)t_q, (int)t_kv, gw, (int)grid.x, q, (int)ldq, k,
-                       (int)ldk, v, (int)ldv, out, (int)ldo, part, P, nullptr, 0, BeamCaches{});
-  else if (rows)
-    hipLaunchKernelGGL((k_attn<true, 2>), grid, dim3(128), 0, s, (int)t_q, (int)t_kv, gw, (int)grid.x, q, (int)ldq, k,
-                       (int)ldk, v, (int)ldv, out, (int)ldo, part, P, nullptr, 0, BeamCaches{});
-  else if (one_tile)
-    hipLaunchKernelGGL((k_attn<false, 1>), grid, dim3(128), 0, s, (int)t_q, (int)t_kv, gw, (int)grid.x, q, (int)ldq,
-                       nullptr, 0, nullptr, 0, out, (int)ldo, part, P, nullptr, 0, BeamCaches{});
+  const dim3 grid(1u, (unsigned)n_head, (unsigned)nsplit);
+  const int gw = (causal ? 1 : 0) | nsplit << 1 | n_head << 8;  // k_attn's packed grid
+  if (rows)
+    hipLaunchKernelGGL((k_attn<true>), grid, dim3(128), 0, s, (int)t_q, (int)t_kv, gw, 1, q, (int)ldq, k, (int)ldk, v,
+                       (int)ldv, out, (int)ldo, part, P, nullptr, 0, BeamCaches{});
   else
-    hipLaunchKernelGGL((k_attn<false, 2>), grid, dim3(128), 0, s, (int)t_q, (int)t_kv, gw, (int)grid.x, q, (int)ldq,
-                       nullptr, 0, nullptr, 0, out, (int)ldo, part, P, nullptr, 0, BeamCaches{});
+    hipLaunchKernelGGL((k_attn<false>), grid, dim3(128), 0, s, (int)t_q, (int)t_kv, gw, 1, q, (int)ldq, nullptr, 0,
+                       nullptr, 0, out, (int)ldo, part, P, nullptr, 0, BeamCaches{});
   LAUNCH_TRY("k_attn");
   if (part) {
     const size_t nz = t_q * (size_t)n_head * ATT_DH;
@@ -1136,15 +1135,14 @@ struct CrossKV {
   int device = -1;
   size_t n_audio = 0, n = 0;
   int n_layer = 0, tkv_pad = 0;
-  void *buf = nullptr;  // per layer: kh, kl, vh, vl planes of (n_head x 64) x tkv_pad f16
-  size_t layer_bytes = 0, plane_bytes = 0;
+  void *buf = nullptr;  // per layer: [head][tkv_pad / 32][ATT_BLK] f16
+  size_t layer_bytes = 0;
   ~CrossKV() {
     if (buf) (void)hipFree(buf);
   }
   AttnPlanes planes(int l) const {
     const char *b = (const char *)buf + (size_t)l * layer_bytes;
-    return AttnPlanes{nullptr, nullptr, (const uint16_t *)b, (const uint16_t *)(b + plane_bytes),
-                      (const uint16_t *)(b + 2 * plane_bytes), (const uint16_t *)(b + 3 * plane_bytes), 0, tkv_pad};
+    return AttnPlanes{(const uint16_t *)b, 0, tkv_pad};
   }
 };
 
@@ -1237,9 +1235,7 @@ static int run_beam_self_attention(rw_decoder *const *beams, size_t nb, int l, c
   const int n_head = d->p.n_head, heads = (int)nb * n_head;
   const size_t n_past = d->n_past, t_kv = n_past + 1;
   char *b = (char *)ws;
-  AttnPlanes P{(uint16_t *)(b + L.off_qh), (uint16_t *)(b + L.off_ql), (uint16_t *)(b + L.off_kh),
-               (uint16_t *)(b + L.off_kl), (uint16_t *)(b + L.off_vh), (uint16_t *)(b + L.off_vl), L.tq_pad,
-               (int)std::min<size_t>(align_up(t_kv, ATT_KVB), L.tkv_pad)};
+  AttnPlanes P{nullptr, L.tq_pad, (int)std::min<size_t>(align_up(t_kv, ATT_KVB), L.tkv_pad)};
   BeamCaches C{};
   for (size_t i = 0; i < nb; ++i) {
     C.k[i] = beams[i]->self_k(l);
@@ -1251,7 +1247,7 @@ static int run_beam_self_attention(rw_decoder *const *beams, size_t nb, int l, c
   const int nsplit = std::min(L.nsplit, attn_nsplit((size_t)(L.tq_pad / ATT_QB) * heads, cdiv(t_kv, ATT_KVB)));
   float *part = nsplit > 1 ? (float *)(b + L.off_part) : nullptr;
   const bool with_rec = rec && !part && nb >= 2 && nb <= (size_t)GEMV_MAX_M;
-  hipLaunchKernelGGL((k_attn<true, 1, true>), dim3(1, (unsigned)heads, (unsigned)nsplit), dim3(128), 0, s, 1,
+  hipLaunchKernelGGL((k_attn<true, true>), dim3(1, (unsigned)heads, (unsigned)nsplit), dim3(128), 0, s, 1,
                      (int)t_kv, 1 | nsplit << 1 | heads << 8, 1, q, (int)d->n, kn, (int)d->n, vn, (int)d->n, att,
                      (int)d->n, part, P, with_rec ? rec : nullptr, n_head | rec_off << 8 | (int)nb << 16, C);
   LAUNCH_TRY("k_attn");
@@ -2119,8 +2115,7 @@ int rw_rocm_decoder_create(const rw_decoder_params *params, size_t n_audio_ctx, 
   cross->n = d->n;
   cross->n_layer = params->n_layer;
   cross->tkv_pad = (int)align_up(n_audio_ctx, ATT_KVB);
-  cross->plane_bytes = align_up((size_t)params->n_head * ATT_DH * cross->tkv_pad * 2, 256);
-  cross->layer_bytes = 4 * cross->plane_bytes;
+  cross->layer_bytes = (size_t)params->n_head * (cross->tkv_pad / ATT_KVB) * ATT_BLK * 2;
   if (hipMalloc(&cross->buf, cross->layer_bytes * params->n_layer) != hipSuccess) {
     (void)hipGetLastError();
     cross->buf = nullptr;
@@ -2156,7 +2151,6 @@ int rw_rocm_decoder_set_audio_dev(rw_decoder *d, const float *enc_out, void *str
   hipStream_t s = (hipStream_t)stream;
   const size_t T = d->n_audio, n = d->n;
   // k and v f32 for one layer, the activation workspace, then splitting
-  const AttnLayout A = attn_layout(1, T, n);
   const size_t off_k = 0, off_v = align_up(T * n * 4, 256), off_act = align_up(off_v + T * n * 4, 256);
   const size_t bytes = align_up(off_act + act_layout(T, n).bytes, 256);
   int rc = dec_reserve(d, bytes);
@@ -2181,12 +2175,7 @@ int rw_rocm_decoder_set_audio_dev(rw_decoder *d, const float *enc_out, void *str
       RW_TRY(run_product(L.cv, T, L.cv_b, vf, b + off_act, s));
     }
     const AttnPlanes cp = d->cross->planes(l);
-    AttnPlanes P{nullptr, nullptr, cp.kh, cp.kl, cp.vh, cp.vl, A.tq_pad, cp.tkv_pad};
-    const size_t nk = (size_t)d->p.n_head * cp.tkv_pad * 8;
-    const int wk = (int)cdiv(nk, 256), wv = d->p.n_head * (int)cdiv(cp.tkv_pad, ATT_VT_KV);
-    hipLaunchKernelGGL(k_attn_split, dim3((unsigned)(wk + wv)), dim3(256), 0, s, nullptr, (int)n, 0, kf, (int)n, vf,
-                       (int)n, (int)T, P, d->p.n_head, 0, wk);
-    LAUNCH_TRY("k_attn_split");
+    RW_TRY(launch_attn_split(kf, n, vf, n, T, d->p.n_head, const_cast<uint16_t *>(cp.kv), cp.tkv_pad / ATT_KVB, s));
   }
   d->audio = true;
   d->n_past = 0;

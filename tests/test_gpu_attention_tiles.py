@@ -1,0 +1,59 @@
+"""Edges of the attention kernels' dispatch (rw_attn.hpp, run_attention): at
+most 8 query rows (k_attn), 9 to 64 rows (k_attn_tile splitting K and V
+itself), more (from split blocks), 32 or 64 query rows per workgroup; and
+scores that move the softmax's reference exponent in every block.
+
+Bar: 1e-5 of the row's L2 norm against the float64 oracle (operands keep 22
+bits, sums are f32: a few 2^-22 over scores of magnitude s, times s)."""
+import numpy as np
+import pytest
+
+from oracle.attention import mha
+from rusty_whisper_amd import _abi as A
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _device():
+    A.init(0)
+
+
+def err(got, q, k, v, heads, causal):
+    ref = mha(q, k, v, heads, causal, dtype=np.float64)
+    den = np.maximum(np.linalg.norm(ref, axis=1), 1e-30)
+    return float(np.max(np.max(np.abs(got.astype(np.float64) - ref), axis=1) / den))
+
+
+@pytest.mark.parametrize("t_q,t_kv,heads,causal", [
+    (8, 33, 2, True), (9, 9, 2, True), (9, 31, 2, False), (32, 129, 1, True), (33, 33, 2, True), (64, 97, 2, True),
+    (65, 65, 2, True), (65, 160, 3, False), (1030, 70, 24, False), (1030, 1030, 24, True)], ids=str)
+def test_dispatch_edges(t_q, t_kv, heads, causal):
+    rng = np.random.default_rng(t_q + t_kv)
+    q, k, v = (rng.standard_normal((t, 64 * heads)).astype(np.float32) for t in (t_q, t_kv, t_kv))
+    assert err(A.attention(q, k, v, heads, causal), q, k, v, heads, causal) <= 1e-5
+
+
+def test_rows_do_not_depend_on_the_tile():
+    """One query row's result is the same bits from 64-row tiles, 32-row tiles
+    and tiles that split K and V themselves."""
+    rng = np.random.default_rng(3)
+    q, k, v = (rng.standard_normal((t, 64 * 24)).astype(np.float32) for t in (1030, 300, 300))
+    full = A.attention(q, k, v, 24, False)
+    for t in (100, 64, 9):
+        assert np.array_equal(A.attention(q[:t], k, v, 24, False).view(np.uint32), full[:t].view(np.uint32)), t
+
+
+@pytest.mark.parametrize("t_q", [8, 40, 1030])
+@pytest.mark.parametrize("step", [6.0, -6.0, 40.0])
+def test_moving_maxima(t_q, step):
+    """Scores that rise (or fall) by `step` per key, over blocks of every
+    wavefront: each new block moves the reference exponent, or none does."""
+    heads, t_kv = 24, 140
+    rng = np.random.default_rng(int(step) + t_q)
+    q = np.zeros((t_q, 64 * heads), np.float32)
+    k = (rng.standard_normal((t_kv, 64 * heads)) * 0.1).astype(np.float32)
+    v = rng.standard_normal((t_kv, 64 * heads)).astype(np.float32)
+    q[:, ::64] = 8.0  # score = the key's first value
+    k[:, ::64] = (step * np.arange(t_kv, dtype=np.float32))[:, None]
+    assert err(A.attention(q, k, v, heads, False), q, k, v, heads, False) <= 1e-5
