@@ -367,61 +367,245 @@ __global__ __launch_bounds__(256) void k_repack(const uint8_t *__restrict__ raw,
 // over p < k8 = k - k % 8; the tail k8..k summed from -0.0; the lanes summed
 // from -0.0 in order, plus the tail; then + bias[j] (add_bias,
 // src/tensor.rs:262-272).  So results are bit-identical to the reference's.
-// A workgroup computes a 32 x 32 tile from 32-wide k slices of A and B staged
-// in LDS; each thread owns 2 x 2 outputs.
-__global__ __launch_bounds__(256) void k_matmul_t_f32(const float *__restrict__ a, const float *__restrict__ b,
-                                                      const float *__restrict__ bias, float *__restrict__ c,
-                                                      int m, int n, int k) {
-  __shared__ float As[32][33], Bs[32][33];
+
+// the tail and the lanes' sum of element (arow, brow)
+__device__ inline float dense_finish(const float (&acc)[8], const float *__restrict__ arow,
+                                     const float *__restrict__ brow, int k8, int k, const float *__restrict__ bias,
+                                     int j) {
+  float tail = -0.0f;
+  for (int p = k8; p < k; ++p) tail = __fadd_rn(tail, __fmul_rn(arow[p], brow[p]));
+  float s = -0.0f;
+#pragma unroll
+  for (int l = 0; l < 8; ++l) s = __fadd_rn(s, acc[l]);
+  s = __fadd_rn(s, tail);
+  if (bias) s = __fadd_rn(s, bias[j]);
+  return s;
+}
+
+// More than 8 rows.  A workgroup of 256 threads computes a 16 R x 16 R tile
+// from 32-wide k slices of A and B in LDS (double-buffered, the next slice's
+// loads in flight meanwhile); each thread owns R x R outputs, rows ty + 16 u and
+// columns tx + 16 v, and reads 8 consecutive k of a row at a time (two 16-byte
+// LDS reads; rows 36 floats apart start on distinct banks).
+// Bound by the VALU: a product and a sum rounded apart are two instructions,
+// 2 m n k / 64 of them at 4 cycles each: 125 us at 2.4 GHz for 1500 x 1280 x
+// 1280 (147 us; R = 2 with 4-byte LDS reads, two per product, took 268; R = 4
+// 149, at two wavefronts per SIMD).  R = 1 is for launches that 32-row tiles
+// leave under 512 workgroups: 100 x 384 x 1536 21 against 55 us, 224 x 1280 x
+// 1280 39 against 49, but 1500 x 384 x 384 (564 tiles) 21.5 against 20.8.  VEC:
+// rows start on 16 bytes.
+constexpr int DENSE_KS = 32, DENSE_LD = DENSE_KS + 4;
+template <int R, bool VEC>
+__global__ __launch_bounds__(256, 2) void k_matmul_t_f32(const float *__restrict__ a, const float *__restrict__ b,
+                                                         const float *__restrict__ bias, float *__restrict__ c, int m,
+                                                         int n, int k) {
+  constexpr int T = 16 * R, UQ = R == 1 ? DENSE_KS / 8 : 1;  // rows of a tile side
+  constexpr int NV = T * (DENSE_KS / 4) / 256 ? T * (DENSE_KS / 4) / 256 : 1;  // 16-byte pieces per thread and side
+  constexpr bool HALF = T * (DENSE_KS / 4) < 256;  // a side is half the threads' pieces: A and B together
+  __shared__ __align__(16) float sh[2][2][T * DENSE_LD];
   const int t = threadIdx.x, tx = t & 15, ty = t >> 4;
-  const int i0 = blockIdx.y * 32, j0 = blockIdx.x * 32;
+  const int i0 = blockIdx.y * T, j0 = blockIdx.x * T;
   const int k8 = k - k % 8;
-  float acc[2][2][8];
+  // piece e of this thread: side, row and k of the slice
+  auto piece = [&](int side, int e, int &sd, int &row, int &q) __attribute__((always_inline)) {
+    const int idx = HALF ? (t & 127) : t + 256 * e;
+    sd = HALF ? t >> 7 : side;
+    row = idx >> 3;
+    q = (idx & 7) * 4;
+  };
+  float4 nx[HALF ? 1 : 2][NV];
+  auto load = [&](int p0) __attribute__((always_inline)) {
 #pragma unroll
-  for (int u = 0; u < 2; ++u)
+    for (int side = 0; side < (HALF ? 1 : 2); ++side)
 #pragma unroll
-    for (int v = 0; v < 2; ++v)
+      for (int e = 0; e < NV; ++e) {
+        int sd, row, q;
+        piece(side, e, sd, row, q);
+        const int gr = (sd ? j0 : i0) + row, lim = sd ? n : m, p = p0 + q;
+        const float *src = (sd ? b : a) + (size_t)min(gr, lim - 1) * k;
+        // past k8 (or past m, n) the values are +0, whose products (+0) leave
+        // every accumulator as it is (k8 is a multiple of 4: a piece is in or out)
+        float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (gr < lim && p < k8) {
+          if (VEC) x = *reinterpret_cast<const float4 *>(src + p);
+          else x = make_float4(src[p], src[p + 1], src[p + 2], src[p + 3]);
+        }
+        nx[side][e] = x;
+      }
+  };
+  auto store = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int side = 0; side < (HALF ? 1 : 2); ++side)
+#pragma unroll
+      for (int e = 0; e < NV; ++e) {
+        int sd, row, q;
+        piece(side, e, sd, row, q);
+        *reinterpret_cast<float4 *>(&sh[buf][sd][row * DENSE_LD + q]) = nx[side][e];
+      }
+  };
+  float acc[R][R][8];
+#pragma unroll
+  for (int u = 0; u < R; ++u)
+#pragma unroll
+    for (int v = 0; v < R; ++v)
 #pragma unroll
       for (int l = 0; l < 8; ++l) acc[u][v][l] = 0.0f;
-  for (int p0 = 0; p0 < k8; p0 += 32) {
-    // 4 values per thread per tile; past k8 (or past m, n) they are +0, whose
-    // products (+0) leave every accumulator as it is
+  load(0);
+  store(0);
+  __syncthreads();
+  int buf = 0;
+  for (int p0 = 0; p0 < k8; p0 += DENSE_KS, buf ^= 1) {
+    const bool more = p0 + DENSE_KS < k8;  // uniform
+    if (more) load(p0 + DENSE_KS);
+    const float *As = sh[buf][0], *Bs = sh[buf][1];
+#pragma unroll UQ  // (R = 2: the operands of all four steps at once cost more than the loop)
+    for (int q0 = 0; q0 < DENSE_KS; q0 += 8) {
+      float bv[R][8];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int idx = t + 256 * e, r = idx >> 5, q = idx & 31, p = p0 + q;
-      As[r][q] = (i0 + r < m && p < k8) ? a[(size_t)(i0 + r) * k + p] : 0.0f;
-      Bs[r][q] = (j0 + r < n && p < k8) ? b[(size_t)(j0 + r) * k + p] : 0.0f;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int q0 = 0; q0 < 32; q0 += 8)
-#pragma unroll
-      for (int l = 0; l < 8; ++l) {
-        const float a0 = As[2 * ty][q0 + l], a1 = As[2 * ty + 1][q0 + l];
-        const float b0 = Bs[2 * tx][q0 + l], b1 = Bs[2 * tx + 1][q0 + l];
-        acc[0][0][l] = __fadd_rn(acc[0][0][l], __fmul_rn(a0, b0));
-        acc[0][1][l] = __fadd_rn(acc[0][1][l], __fmul_rn(a0, b1));
-        acc[1][0][l] = __fadd_rn(acc[1][0][l], __fmul_rn(a1, b0));
-        acc[1][1][l] = __fadd_rn(acc[1][1][l], __fmul_rn(a1, b1));
+      for (int v = 0; v < R; ++v) {
+        *reinterpret_cast<float4 *>(&bv[v][0]) = *reinterpret_cast<const float4 *>(&Bs[(tx + 16 * v) * DENSE_LD + q0]);
+        *reinterpret_cast<float4 *>(&bv[v][4]) =
+            *reinterpret_cast<const float4 *>(&Bs[(tx + 16 * v) * DENSE_LD + q0 + 4]);
       }
+#pragma unroll
+      for (int u = 0; u < R; ++u) {
+        float av[8];
+        *reinterpret_cast<float4 *>(&av[0]) = *reinterpret_cast<const float4 *>(&As[(ty + 16 * u) * DENSE_LD + q0]);
+        *reinterpret_cast<float4 *>(&av[4]) = *reinterpret_cast<const float4 *>(&As[(ty + 16 * u) * DENSE_LD + q0 + 4]);
+#pragma unroll
+        for (int v = 0; v < R; ++v)
+#pragma unroll
+          for (int l = 0; l < 8; ++l) acc[u][v][l] = __fadd_rn(acc[u][v][l], __fmul_rn(av[l], bv[v][l]));
+      }
+    }
+    if (more) store(buf ^ 1);  // that buffer's readers passed the last barrier
     __syncthreads();
   }
 #pragma unroll
-  for (int u = 0; u < 2; ++u)
+  for (int u = 0; u < R; ++u)
 #pragma unroll
-    for (int v = 0; v < 2; ++v) {
-      const int i = i0 + 2 * ty + u, j = j0 + 2 * tx + v;
-      if (i < m && j < n) {
-        float tail = -0.0f;
-        for (int p = k8; p < k; ++p) tail = __fadd_rn(tail, __fmul_rn(a[(size_t)i * k + p], b[(size_t)j * k + p]));
-        float s = -0.0f;
+    for (int v = 0; v < R; ++v) {
+      const int i = i0 + ty + 16 * u, j = j0 + tx + 16 * v;
+      if (i < m && j < n) c[(size_t)i * n + j] = dense_finish(acc[u][v], a + (size_t)i * k, b + (size_t)j * k, k8, k, bias, j);
+    }
+}
+
+// orders one wavefront's LDS accesses (which complete in order) for the
+// compiler; no wait, unlike a barrier, which would also wait for every load in
+// flight
+__device__ inline void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// At most 8 rows (a decoding step).  One wavefront per 8 weight rows: 8 lanes
+// per row, lane l the l-th accumulator of each of the M activation rows, whose
+// terms run down k one after another.  The rows stream in as 128-byte pieces (8
+// lanes, 32 k; PD of them in flight per row) and pass through LDS to the lanes
+// that sum them, U pieces at a time; the activations of PD pieces, requested a
+// chunk ahead, sit in LDS by accumulator, so a lane reads 4 steps' values at
+// once.  Bound by HBM for large weights (51866 x 1280: 40 us, 6.7 TB/s), else by
+// a memory round trip and the chain of sums (2048 x 512 3.4 us, against 34 in
+// 32-row tiles; 1280 x 5120 15 us; branches around the loads, which made every
+// round wait for all of them, 23 us).
+template <int M, bool VEC>
+__global__ __launch_bounds__(64, 1) void k_matvec_t_f32(const float *__restrict__ a, const float *__restrict__ b,
+                                                        const float *__restrict__ bias, float *__restrict__ c, int n,
+                                                        int k) {
+  constexpr int PD = 16, U = 4, SC = 4 * PD, NX = PD / 2;  // steps and activations (64 lanes) per chunk
+  constexpr int XLD = SC + 4, WLD = 40;                    // accumulators and rows start on distinct banks
+  __shared__ __align__(16) float xs[M][8][XLD];
+  __shared__ __align__(16) float ws[U][8][WLD];
+  const int t = threadIdx.x, l = t & 7, r = t >> 3;
+  const int j = blockIdx.x * 8 + r;
+  const float *brow = b + (size_t)min(j, n - 1) * k;
+  const int k8 = k - k % 8, groups = (k8 + 31) / 32;  // pieces of 32 k
+  // past k8 weights and activations are +0, whose products (+0) leave every
+  // accumulator as it is
+  auto piece = [&](int g) __attribute__((always_inline)) {
+    const int p = 32 * g + 4 * l, q = min(p, k8 - 4);  // (no branch: it would wait for every load in flight)
+    float4 x;
+    if (VEC) x = *reinterpret_cast<const float4 *>(brow + q);
+    else x = make_float4(brow[q], brow[q + 1], brow[q + 2], brow[q + 3]);
+    return x;
+  };
+  // the pieces' values past k8 to +0 (the last piece of a row, or a refill past it)
+  auto live = [&](int g, float4 x) __attribute__((always_inline)) {
+    const bool in = 32 * g + 4 * l < k8;
+    return make_float4(in ? x.x : 0.f, in ? x.y : 0.f, in ? x.z : 0.f, in ? x.w : 0.f);
+  };
+  float xr[M][NX];
+  auto load_x = [&](int g0) __attribute__((always_inline)) {
 #pragma unroll
-        for (int l = 0; l < 8; ++l) s = __fadd_rn(s, acc[u][v][l]);
-        s = __fadd_rn(s, tail);
-        if (bias) s = __fadd_rn(s, bias[j]);
-        c[(size_t)i * n + j] = s;
+    for (int i = 0; i < M; ++i)
+#pragma unroll
+      for (int e = 0; e < NX; ++e) {
+        const int p = 32 * g0 + 64 * e + t;
+        xr[i][e] = a[(size_t)i * k + min(p, k8 - 1)];
+      }
+  };
+  float acc[M];
+#pragma unroll
+  for (int i = 0; i < M; ++i) acc[i] = 0.0f;
+  if (k8) {  // uniform
+    float4 w[PD];
+    load_x(0);
+#pragma unroll
+    for (int u = 0; u < PD; ++u) w[u] = piece(u);
+    // round v of a chunk: pieces v .. v + U - 1 into LDS, their ring slots
+    // refilled, and this lane's column of them requested from LDS
+    float wv[2][U][4];
+    auto pass = [&](int g0, int v, float (&o)[U][4]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        *reinterpret_cast<float4 *>(&ws[u][r][4 * l]) = live(g0 + v + u, w[v + u]);
+        w[v + u] = piece(g0 + v + u + PD);
+      }
+      wave_lds_fence();
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[u][e] = ws[u][r][8 * e + l];
+      wave_lds_fence();
+    };
+    pass(0, 0, wv[0]);
+    for (int g0 = 0; g0 < groups; g0 += PD) {
+#pragma unroll
+      for (int i = 0; i < M; ++i)
+#pragma unroll
+        for (int e = 0; e < NX; ++e) xs[i][t & 7][8 * e + (t >> 3)] = 32 * g0 + 64 * e + t < k8 ? xr[i][e] : 0.0f;
+      load_x(g0 + PD);
+      wave_lds_fence();
+#pragma unroll
+      for (int v = 0; v < PD; v += U) {
+        if (g0 + v < groups) {  // uniform
+          // the next round's weights pass through LDS while this one's are summed
+          const int cur = (v / U) & 1;
+          if (v + U < PD) pass(g0, v + U, wv[cur ^ 1]);
+          else pass(g0 + PD, 0, wv[cur ^ 1]);
+#pragma unroll
+          for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int i = 0; i < M; ++i) {
+              const float4 x = *reinterpret_cast<const float4 *>(&xs[i][l][4 * (v + u)]);
+              acc[i] = __fadd_rn(acc[i], __fmul_rn(x.x, wv[cur][u][0]));
+              acc[i] = __fadd_rn(acc[i], __fmul_rn(x.y, wv[cur][u][1]));
+              acc[i] = __fadd_rn(acc[i], __fmul_rn(x.z, wv[cur][u][2]));
+              acc[i] = __fadd_rn(acc[i], __fmul_rn(x.w, wv[cur][u][3]));
+            }
+          wave_lds_fence();
+        }
       }
     }
+  }
+#pragma unroll
+  for (int i = 0; i < M; ++i) {
+    float lanes[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) lanes[e] = __shfl(acc[i], (t & ~7) + e);
+    if (l == 0 && j < n) c[(size_t)i * n + j] = dense_finish(lanes, a + (size_t)i * k, brow, k8, k, bias, j);
+  }
 }
 
 // -------------------------------------------------------------- k_dequant

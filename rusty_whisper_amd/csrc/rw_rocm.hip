@@ -1777,8 +1777,41 @@ static int check_dense_args(const float *a, size_t m, size_t k, const float *b, 
 
 static int launch_matmul_t_f32(const float *a, size_t m, size_t k, const float *b, size_t n, const float *bias,
                                float *out, hipStream_t s) {
-  hipLaunchKernelGGL(k_matmul_t_f32, dim3((unsigned)cdiv(n, 32), (unsigned)cdiv(m, 32)), dim3(256), 0, s, a, b, bias,
-                     out, (int)m, (int)n, (int)k);
+  const bool vec = k % 4 == 0 && al16(a) && al16(b);  // every row starts on 16 bytes
+  // at most 8 rows: by weight rows (k_matvec_t_f32 indexes k in ints, with
+  // up to two chunks past the end)
+  if (m <= 8 && k <= (size_t)1 << 30) {
+    const dim3 grid((unsigned)cdiv(n, 8));
+#define RW_VEC(M)                                                                                                      \
+  case M:                                                                                                              \
+    if (vec) hipLaunchKernelGGL((k_matvec_t_f32<M, true>), grid, dim3(64), 0, s, a, b, bias, out, (int)n, (int)k);     \
+    else hipLaunchKernelGGL((k_matvec_t_f32<M, false>), grid, dim3(64), 0, s, a, b, bias, out, (int)n, (int)k);        \
+    break
+    switch (m) {
+      RW_VEC(1);
+      RW_VEC(2);
+      RW_VEC(3);
+      RW_VEC(4);
+      RW_VEC(5);
+      RW_VEC(6);
+      RW_VEC(7);
+      RW_VEC(8);
+    }
+#undef RW_VEC
+    LAUNCH_TRY("k_matvec_t_f32");
+    return RW_OK;
+  }
+  // 32 x 32 tiles where they make 512 workgroups, two per CU, else 16 x 16
+  // (k_matmul_t_f32 has both sides measured)
+  const int R = cdiv(n, 32) * cdiv(m, 32) >= 512 ? 2 : 1;
+  const dim3 grid((unsigned)cdiv(n, 16 * R), (unsigned)cdiv(m, 16 * R));
+#define RW_DENSE(R, V)                                                                                               \
+  hipLaunchKernelGGL((k_matmul_t_f32<R, V>), grid, dim3(256), 0, s, a, b, bias, out, (int)m, (int)n, (int)k)
+  if (R == 2 && vec) RW_DENSE(2, true);
+  else if (R == 2) RW_DENSE(2, false);
+  else if (vec) RW_DENSE(1, true);
+  else RW_DENSE(1, false);
+#undef RW_DENSE
   LAUNCH_TRY("k_matmul_t_f32");
   return RW_OK;
 }
