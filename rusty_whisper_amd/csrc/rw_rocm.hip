@@ -430,21 +430,22 @@ static void launch_gemm_tm(const GemmSet &set, size_t tiles, const ActView &av, 
 #ifndef GEMM_TN1_BELOW
 #define GEMM_TN1_BELOW 512
 #endif
+// (the launch's column tiles of tn weight row groups each; their starts to set)
+static size_t gemm_column_tiles(GemmSet &set, int tn) {
+  size_t t = 0;
+  for (int i = 0; i < set.count; ++i) {
+    set.it[i].tile0 = (int)t;
+    t += cdiv((size_t)set.it[i].ngroups, (size_t)tn);
+  }
+  return t;
+}
 template <int DT, int KW, bool OFFS>
 static bool launch_gemm_narrow(GemmSet set, size_t tiles, const ActView &av, int m, hipStream_t s) {
   if (cdiv(av.mgroups, 2) * tiles * KW >= GEMM_TN1_BELOW) return false;
-  size_t t1 = 0;
-  for (int i = 0; i < set.count; ++i) {
-    set.it[i].tile0 = (int)t1;
-    t1 += (size_t)set.it[i].ngroups;
-  }
-  launch_gemm_tm<DT, KW, 2, OFFS, 1>(set, t1, av, m, s);
+  launch_gemm_tm<DT, KW, 2, OFFS, 1>(set, gemm_column_tiles(set, 1), av, m, s);
   return true;
 }
 
-// A single-wavefront launch whose 128-row tiles leave SIMDs idle takes
-// 96-row tiles when those still fit one wavefront per SIMD (q/k/v of a
-// 1500-row input: 720 wavefronts of 128 rows, or 960 of 96, on 1024 SIMDs).
 // A launch that 128-row tiles would give fewer than GEMM_TM2_BELOW
 // wavefronts (a skinny input: a 224-row prompt's products run 120-160)
 // takes 64-row tiles, twice the wavefronts (the 32 large-v3 layers'
@@ -454,31 +455,50 @@ constexpr size_t GEMM_SIMDS = 1024;
 #ifndef GEMM_TM2_BELOW
 #define GEMM_TM2_BELOW 512
 #endif
-static int gemm_rows(int kw, size_t tiles, int mgroups) {
-  if (mgroups <= 2) return 2;
-  if (cdiv(mgroups, 4) * tiles * kw < GEMM_TM2_BELOW) return 2;
-  if (kw == 1 && cdiv(mgroups, 3) * tiles <= GEMM_SIMDS && cdiv(mgroups, 4) * tiles < cdiv(mgroups, 3) * tiles)
-    return 3;
-  return 4;
+static bool gemm_skinny(int kw, size_t tiles, int mgroups) {
+  return mgroups <= 2 || cdiv(mgroups, 4) * tiles * kw < GEMM_TM2_BELOW;
 }
 
+// The tile of a single-wavefront launch: 128 x 64, 96 x 64 or 96 x 128,
+// whichever needs the least time as rounds of one wavefront per SIMD times a
+// tile's own time (100, 80 and 138, from 228, 229 and 197 us in 8, 10 and 5
+// rounds at 12000 x 5120 x 1280).  The other launches measured follow it: 1500
+// x 3840 x 1280 23.6, 21.0, 30.0 us in one round each; 1500 x 5120 26.2, 34.2
+// (2 rounds), 31.9; 6000 x 3072 x 768 49.5, 42.8, 45.7 in 3, 3 and 2.  The
+// widest tile only without offset rows (their epilogue values would not fit
+// the registers beside it).
+struct GemmTile {
+  int tm, tn;
+};
+static GemmTile gemm_tile_rule(size_t tiles, size_t wide_tiles, int mgroups, bool offs) {
+  auto time = [&](int tm, size_t cols, size_t t) { return cdiv(cdiv((size_t)mgroups, (size_t)tm) * cols, GEMM_SIMDS) * t; };
+  const size_t t42 = time(4, tiles, 100), t32 = time(3, tiles, 80), t34 = time(3, wide_tiles, 138);
+  if (!offs && t34 < t42 && t34 < t32) return {3, 4};
+  return t32 < t42 ? GemmTile{3, 2} : GemmTile{4, 2};
+}
+
+template <int DT, int KW, bool OFFS>
+static void launch_gemm_offs(const GemmSet &set, size_t tiles, const ActView &av, int m, hipStream_t s) {
+  if (gemm_skinny(KW, tiles, av.mgroups)) {
+    if (!launch_gemm_narrow<DT, KW, OFFS>(set, tiles, av, m, s)) launch_gemm_tm<DT, KW, 2, OFFS>(set, tiles, av, m, s);
+    return;
+  }
+  if constexpr (KW == 1) {
+    GemmSet wide = set;
+    const size_t wide_tiles = gemm_column_tiles(wide, 4);
+    const GemmTile t = gemm_tile_rule(tiles, wide_tiles, av.mgroups, OFFS);
+    if constexpr (!OFFS)
+      if (t.tn == 4) return launch_gemm_tm<DT, 1, 3, false, 4>(wide, wide_tiles, av, m, s);
+    if (t.tm == 3) return launch_gemm_tm<DT, 1, 3, OFFS>(set, tiles, av, m, s);
+  }
+  launch_gemm_tm<DT, KW, 4, OFFS>(set, tiles, av, m, s);
+}
 template <int DT, int KW>
 static void launch_gemm_kw(const GemmSet &set, size_t tiles, const ActView &av, int m, hipStream_t s) {
   bool offs = false;
   for (int i = 0; i < set.count; ++i) offs = offs || set.it[i].gp.cm != nullptr;
-  const int tm = gemm_rows(KW, tiles, av.mgroups);
-  if (tm == 2 && (offs ? launch_gemm_narrow<DT, KW, true>(set, tiles, av, m, s)
-                      : launch_gemm_narrow<DT, KW, false>(set, tiles, av, m, s)))
-    return;
-  if (offs) {
-    if (tm == 2) launch_gemm_tm<DT, KW, 2, true>(set, tiles, av, m, s);
-    else if (KW == 1 && tm == 3) launch_gemm_tm<DT, 1, 3, true>(set, tiles, av, m, s);
-    else launch_gemm_tm<DT, KW, 4, true>(set, tiles, av, m, s);
-  } else {
-    if (tm == 2) launch_gemm_tm<DT, KW, 2, false>(set, tiles, av, m, s);
-    else if (KW == 1 && tm == 3) launch_gemm_tm<DT, 1, 3, false>(set, tiles, av, m, s);
-    else launch_gemm_tm<DT, KW, 4, false>(set, tiles, av, m, s);
-  }
+  if (offs) launch_gemm_offs<DT, KW, true>(set, tiles, av, m, s);
+  else launch_gemm_offs<DT, KW, false>(set, tiles, av, m, s);
 }
 
 template <int DT>
