@@ -154,44 +154,60 @@ __global__ __launch_bounds__(256) void k_topk_stats(const float *__restrict__ lo
   }
 }
 
+// A wavefront's largest value and smallest int, by DPP row moves (a lane
+// without a source keeps its own value), the same in every lane.
+template <int CTRL, int ROWS = 0xf>
+__device__ inline int topk_dpp(int v) {
+  return __builtin_amdgcn_update_dpp(v, v, CTRL, ROWS, 0xf, false);
+}
+__device__ inline float wave_fmax(float v) {
+  auto up = [&](int o) __attribute__((always_inline)) { v = fmaxf(v, __int_as_float(o)); };
+  up(topk_dpp<0x111>(__float_as_int(v)));       // row_shr 1, 2, 4, 8
+  up(topk_dpp<0x112>(__float_as_int(v)));
+  up(topk_dpp<0x114>(__float_as_int(v)));
+  up(topk_dpp<0x118>(__float_as_int(v)));
+  up(topk_dpp<0x142, 0xa>(__float_as_int(v)));  // row_bcast 15 into rows 1 and 3
+  up(topk_dpp<0x143, 0xc>(__float_as_int(v)));  // row_bcast 31 into rows 2 and 3
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+}
+__device__ inline int wave_imin(int v) {
+  v = min(v, topk_dpp<0x111>(v));
+  v = min(v, topk_dpp<0x112>(v));
+  v = min(v, topk_dpp<0x114>(v));
+  v = min(v, topk_dpp<0x118>(v));
+  v = min(v, topk_dpp<0x142, 0xa>(v));
+  v = min(v, topk_dpp<0x143, 0xc>(v));
+  return __builtin_amdgcn_readlane(v, 63);
+}
+
 // the row's lse from its chunks' (maximum, sum) pairs: the maximum of the
-// maxima, then sum_c s_c exp(m_c - M) in chunk order.  A chunk of NaNs only
-// (maximum -inf, sum NaN) still makes it NaN, and so does a row of -inf
-// only, whose reference maximum -inf gives -inf - -inf = NaN.
+// maxima, then sum_c s_c exp(m_c - M) in chunk order (one chunk per lane, at
+// most 64; every wavefront computes it).  A chunk of NaNs only (maximum -inf,
+// sum NaN) still makes it NaN, and so does a row of -inf only, whose reference
+// maximum -inf gives -inf - -inf = NaN.
 __device__ inline float topk_lse(const float *pm, const float *ps, int nc) {
-  float M = -__builtin_huge_valf();
-  for (int c = 0; c < nc; ++c) M = fmaxf(M, pm[c]);
+  const int l = threadIdx.x & 63;
+  const float m = l < nc ? pm[l] : -__builtin_huge_valf(), s = l < nc ? ps[l] : 0.0f;
+  const float M = wave_fmax(m);
   if (M == -__builtin_huge_valf()) return __builtin_nanf("");
+  const float term = s * expf(m - M);
+  const uint64_t live = __builtin_amdgcn_ballot_w64(m > -__builtin_huge_valf() || s != s);
   float S = 0.0f;
-  for (int c = 0; c < nc; ++c)
-    if (pm[c] > -__builtin_huge_valf() || ps[c] != ps[c]) S += ps[c] * expf(pm[c] - M);
+  for (int c = 0; c < nc; ++c) {
+    const float t = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(term), c));
+    if (live >> c & 1) S += t;
+  }
   return M + logf(S);
 }
 
-// the block-wide first (v, i) in the selection order (lp desc, id asc)
-__device__ inline void block_topk_argmax(float &bv, int &bi, float *rv, int *ri) {
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const float ov = __shfl_xor(bv, o);
-    const int oi = __shfl_xor(bi, o);
-    if (topk_before(ov, oi, bv, bi)) bv = ov, bi = oi;
-  }
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) rv[threadIdx.x >> 6] = bv, ri[threadIdx.x >> 6] = bi;
-  __syncthreads();
-  bv = rv[0], bi = ri[0];
-#pragma unroll
-  for (int w = 1; w < 4; ++w)
-    if (topk_before(rv[w], ri[w], bv, bi)) bv = rv[w], bi = ri[w];
-}
-
-// k rounds over the values a thread holds (`cnt` of them): each round picks
-// the block's first entry after the previous pick; picks go to (ov, oi)[0, k),
-// padded with (-inf, INT32_MAX).  Returns the number picked.
+// k rounds over the values the lanes of one wavefront hold (PER each): each
+// round picks the wavefront's first entry after the previous pick in the
+// selection order (lp desc, id asc); picks go to (ov, oi)[0, k), padded with
+// (-inf, INT32_MAX).  Returns the number picked (uniform).
 template <int PER>
-__device__ inline int topk_rounds(const float (&lp)[PER], const int (&id)[PER], int k, float *ov, int *oi,
-                                  float *rv, int *ri) {
+__device__ inline int topk_rounds(const float (&lp)[PER], const int (&id)[PER], int k, float *ov, int *oi) {
   constexpr float NEG_INF = -__builtin_huge_valf();
+  const bool first = (threadIdx.x & 63) == 0;
   float pv = __builtin_huge_valf();
   int pi = -1, got = 0;
   for (int r = 0; r < k; ++r) {
@@ -201,22 +217,50 @@ __device__ inline int topk_rounds(const float (&lp)[PER], const int (&id)[PER], 
     for (int j = 0; j < PER; ++j)
       if (lp[j] > NEG_INF && topk_before(pv, pi, lp[j], id[j]) && topk_before(lp[j], id[j], bv, bi))
         bv = lp[j], bi = id[j];
-    block_topk_argmax(bv, bi, rv, ri);
-    if (bi == INT32_MAX) break;  // no candidate left (uniform)
-    if (threadIdx.x == 0) ov[r] = bv, oi[r] = bi;
-    pv = bv, pi = bi;
+    const float mv = wave_fmax(bv);
+    const int mi = wave_imin(bv == mv ? bi : INT32_MAX);
+    if (mi == INT32_MAX) break;  // no candidate left (uniform)
+    if (first) ov[r] = mv, oi[r] = mi;
+    pv = mv, pi = mi;
     got = r + 1;
   }
-  if (threadIdx.x == 0)
+  if (first)
     for (int r = got; r < k; ++r) ov[r] = NEG_INF, oi[r] = INT32_MAX;
   return got;
+}
+
+// The first k entries of the values that the 256 threads hold, to (ov, oi) by
+// wavefront 0 (the return value is wavefront 0's): each wavefront's first k
+// into LDS without a barrier, then wavefront 0's rounds over those 4 k.  The
+// entries, and their order, are the block's (a barrier-free round takes about
+// 0.15 us; block-wide arg-max rounds, two barriers and 12 lane shuffles each,
+// took 18 us per launch over 26 chunks of 5 rows with k = 5, and 12 us in the
+// merge).
+constexpr int TOPK_CAND = 2 * TOPK_MAX - 1;  // entries kept per chunk at most
+template <int PER, int KMAX>
+__device__ inline int topk_block(const float (&lp)[PER], const int (&id)[PER], int k, float *ov, int *oi,
+                                 float (&sv)[4 * KMAX], int (&si)[4 * KMAX]) {
+  constexpr int PW = (4 * KMAX + 63) / 64;
+  const int wv = threadIdx.x >> 6, l = threadIdx.x & 63;
+  topk_rounds<PER>(lp, id, k, sv + wv * k, si + wv * k);
+  __syncthreads();
+  if (wv) return 0;
+  float v[PW];
+  int i[PW];
+#pragma unroll
+  for (int j = 0; j < PW; ++j) {
+    const int e = j * 64 + l;
+    v[j] = e < 4 * k ? sv[e] : -__builtin_huge_valf();
+    i[j] = e < 4 * k ? si[e] : INT32_MAX;
+  }
+  return topk_rounds<PW>(v, i, k, ov, oi);
 }
 
 __global__ __launch_bounds__(256) void k_topk_chunk(const float *__restrict__ logits, int n, int k,
                                                     const float *__restrict__ pm, const float *__restrict__ ps,
                                                     float *__restrict__ cv, int *__restrict__ ci) {
-  __shared__ float rv[4];
-  __shared__ int ri[4];
+  __shared__ float sv[4 * TOPK_CAND];
+  __shared__ int si[4 * TOPK_CAND];
   const int c = blockIdx.x, row = blockIdx.y, nc = gridDim.x, t = threadIdx.x;
   const float lse = topk_lse(pm + (size_t)row * nc, ps + (size_t)row * nc, nc);
   const float *x = logits + (size_t)row * n;
@@ -232,7 +276,7 @@ __global__ __launch_bounds__(256) void k_topk_chunk(const float *__restrict__ lo
   }
   const int cand = 2 * k - 1;
   const size_t o = ((size_t)row * nc + c) * cand;
-  topk_rounds<PER>(lp, id, cand, cv + o, ci + o, rv, ri);
+  topk_block<PER, TOPK_CAND>(lp, id, cand, cv + o, ci + o, sv, si);
 }
 
 // the block-wide smallest of one int per thread
@@ -250,8 +294,9 @@ __global__ __launch_bounds__(256) void k_topk_merge(int nc, int k, int n, const 
                                                     const int *__restrict__ ci, uint32_t *__restrict__ ids,
                                                     float *__restrict__ lps) {
   constexpr float NEG_INF = -__builtin_huge_valf();
-  __shared__ float rv[4];
-  __shared__ int ri[4];
+  __shared__ float sv[4 * TOPK_MAX];
+  __shared__ int si[4 * TOPK_MAX];
+  __shared__ int ri[4], n_got;
   __shared__ float pick_v[TOPK_MAX];
   __shared__ int pick_i[TOPK_MAX];
   __shared__ int adm[TOPK_MAX];
@@ -267,7 +312,7 @@ __global__ __launch_bounds__(256) void k_topk_merge(int nc, int k, int n, const 
     }
     return;
   }
-  constexpr int PER = (TOPK_MAX_CHUNKS * (2 * TOPK_MAX - 1) + 255) / 256;
+  constexpr int PER = (TOPK_MAX_CHUNKS * TOPK_CAND + 255) / 256;
   float lp[PER];
   int id[PER];
   const int total = nc * (2 * k - 1);
@@ -279,8 +324,10 @@ __global__ __launch_bounds__(256) void k_topk_merge(int nc, int k, int n, const 
   }
   // the k first in the order (lp desc, id asc): their values are the k
   // largest log-probs, so the last is v*
-  const int got = topk_rounds<PER>(lp, id, k, pick_v, pick_i, rv, ri);
+  const int got0 = topk_block<PER, TOPK_MAX>(lp, id, k, pick_v, pick_i, sv, si);
+  if (t == 0) n_got = got0;
   __syncthreads();
+  const int got = n_got;
   int g = got, a = 0;
   if (got == k) {
     const float vs = pick_v[k - 1];
