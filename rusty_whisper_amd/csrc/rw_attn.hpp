@@ -5,7 +5,8 @@
 //
 //   k_attn_split   k and v (f32) -> f16 pairs x = hi + lo (hi = f16(x), lo =
 //        f16(x - hi)), stored as the matrix cores' operands: per (head, 32 kv
-//        rows) the 16 KB of ATT_BLK below
+//        rows) the 16 KB of ATT_BLK below (k_gemm's GEMM_KOP and GEMM_VOP
+//        epilogues write the same blocks from the products that make K and V)
 //   k_attn_tile    calls of more than 8 query rows: one workgroup per (32 or
 //        64 query rows, head), whose 4 wavefronts split the kv blocks
 //        between them and meet in LDS at the end
@@ -92,12 +93,14 @@ __device__ inline void att_split(float x, uint16_t &hi, uint16_t &lo) {
 }
 
 // 8 f32 values -> the 8 hi and the 8 lo halves
-__device__ inline void att_split8(const float (&v)[8], uint16_t *__restrict__ hi, uint16_t *__restrict__ lo) {
+struct AttSplit8 {
+  uint4 hi, lo;
+};
+__device__ inline AttSplit8 att_split8(const float (&v)[8]) {
   uint16_t h8[8], l8[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) att_split(v[e], h8[e], l8[e]);
-  *reinterpret_cast<uint4 *>(hi) = *reinterpret_cast<const uint4 *>(h8);
-  *reinterpret_cast<uint4 *>(lo) = *reinterpret_cast<const uint4 *>(l8);
+  return {*reinterpret_cast<const uint4 *>(h8), *reinterpret_cast<const uint4 *>(l8)};
 }
 
 // One workgroup per (head, 32-row kv block): its K rows (row-contiguous
@@ -132,8 +135,11 @@ __global__ __launch_bounds__(256) void k_attn_split(const float *__restrict__ k,
     }
   }
   const int ko = ((c >> 1) * 64 + 32 * (c & 1) + n) * 8, vo = 2 * ATT_PART + t * 8;
-  att_split8(kx, o + ko, o + ATT_PART + ko);
-  att_split8(vx, o + vo, o + ATT_PART + vo);
+  const AttSplit8 ks = att_split8(kx), vs = att_split8(vx);
+  *reinterpret_cast<uint4 *>(o + ko) = ks.hi;
+  *reinterpret_cast<uint4 *>(o + ATT_PART + ko) = ks.lo;
+  *reinterpret_cast<uint4 *>(o + vo) = vs.hi;
+  *reinterpret_cast<uint4 *>(o + ATT_PART + vo) = vs.lo;
 }
 
 // Several decoding states' one-token steps in one self-attention: plane

@@ -26,6 +26,7 @@
 #include <hip/hip_runtime.h>
 
 #include "rw_layout.hpp"
+#include "rw_attn.hpp"
 
 namespace rw {
 
@@ -2289,13 +2290,24 @@ constexpr int GEMM_GELU = 1, GEMM_ACC = 2;
 // rows] -- from which k_quantize_finish builds the next product's f16
 // operand (n % 32 == 0)
 constexpr int GEMM_QUANT = 4;
+// GEMM_KOP, GEMM_VOP: the output is an attention layer's K or V (n_head x 64
+// columns, row = kv position), written as k_attn_split would split it instead
+// of in f32: tile (row group, column group) is half of block (head = column
+// group / 2, kv block = row group).  V's fragments are the accumulator's own
+// layout; K's rows go through the wavefront's LDS tile.  The f32 rows, and the
+// launch that split them, leave the encoder layer and the decoder's window
+// (four tiny layers 214 -> 207 us, a large-v3 layer 178 -> 175, set_audio and a
+// 227-token prompt of turbo 588 -> 571).  Not in 128-column tiles, whose
+// registers it would spill (12000 x 5120 x 1280: 202 -> 391 us).
+constexpr int GEMM_KOP = 8, GEMM_VOP = 16;
 struct GemmItem {
   GemmPlanes gp;
   const float *bias;
   float *out;
   int8_t *qo;
   float *ao;
-  int n, ngroups, tile0, flags;
+  uint16_t *kv;  // GEMM_KOP, GEMM_VOP: the layer's operand blocks, kv_nblk per head
+  int n, ngroups, tile0, flags, kv_nblk;
 };
 
 
@@ -2576,6 +2588,41 @@ __device__ __attribute__((always_inline)) inline void gemm_tile(const GemmItem &
           const size_t slot = ((size_t)tg * (size_t)(n / RG) + cg) * RG + rw;
           stg_u32(it.qo + slot * QK + 4 * lt, q);
           if (lt == 0) stg_f(it.ao + slot, amax);
+        }
+      }
+      continue;
+    }
+    if constexpr (TN <= 2) if (flags & (GEMM_KOP | GEMM_VOP)) {
+      uint16_t *blk = it.kv + ((size_t)(cg >> 1) * it.kv_nblk + tg) * ATT_BLK;
+      const int dt = cg & 1;
+      if (flags & GEMM_VOP) {
+        // y[8 s .. 8 s + 7]: rows 16 s + attn_vpos(8 h + e) of value r
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          float v[8];
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            v[e] = tg * RG + 16 * s + attn_vpos(8 * h + e) < m ? y[8 * s + e] : 0.0f;
+          uint16_t *o = blk + 2 * ATT_PART + ((2 * dt + s) * 64 + l) * 8;
+          const AttSplit8 sp = att_split8(v);
+          stg_u4(o, sp.hi);
+          stg_u4(o + ATT_PART, sp.lo);
+        }
+      } else {
+        float *stg = reinterpret_cast<float *>(lds + RED) + kw * (32 * QROW);
+#pragma unroll
+        for (int v = 0; v < 16; ++v) stg[(8 * (v >> 2) + 4 * h + (v & 3)) * QROW + r] = y[v];
+        const bool live = tg * RG + r < m;  // (lane (h, r): row r, values 16 s + 8 h ..)
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          const float4 a = *reinterpret_cast<const float4 *>(stg + r * QROW + 16 * s + 8 * h);
+          const float4 b = *reinterpret_cast<const float4 *>(stg + r * QROW + 16 * s + 8 * h + 4);
+          const float v[8] = {live ? a.x : 0.0f, live ? a.y : 0.0f, live ? a.z : 0.0f, live ? a.w : 0.0f,
+                              live ? b.x : 0.0f, live ? b.y : 0.0f, live ? b.z : 0.0f, live ? b.w : 0.0f};
+          uint16_t *o = blk + ((2 * dt + s) * 64 + l) * 8;
+          const AttSplit8 sp = att_split8(v);
+          stg_u4(o, sp.hi);
+          stg_u4(o + ATT_PART, sp.lo);
         }
       }
       continue;

@@ -465,15 +465,15 @@ static bool gemm_skinny(int kw, size_t tiles, int mgroups) {
 // rounds at 12000 x 5120 x 1280).  The other launches measured follow it: 1500
 // x 3840 x 1280 23.6, 21.0, 30.0 us in one round each; 1500 x 5120 26.2, 34.2
 // (2 rounds), 31.9; 6000 x 3072 x 768 49.5, 42.8, 45.7 in 3, 3 and 2.  The
-// widest tile only without offset rows (their epilogue values would not fit
-// the registers beside it).
+// widest tile only without offset rows or attention operands (their epilogue
+// values would not fit the registers beside it).
 struct GemmTile {
   int tm, tn;
 };
-static GemmTile gemm_tile_rule(size_t tiles, size_t wide_tiles, int mgroups, bool offs) {
+static GemmTile gemm_tile_rule(size_t tiles, size_t wide_tiles, int mgroups, bool wide_ok) {
   auto time = [&](int tm, size_t cols, size_t t) { return cdiv(cdiv((size_t)mgroups, (size_t)tm) * cols, GEMM_SIMDS) * t; };
   const size_t t42 = time(4, tiles, 100), t32 = time(3, tiles, 80), t34 = time(3, wide_tiles, 138);
-  if (!offs && t34 < t42 && t34 < t32) return {3, 4};
+  if (wide_ok && t34 < t42 && t34 < t32) return {3, 4};
   return t32 < t42 ? GemmTile{3, 2} : GemmTile{4, 2};
 }
 
@@ -486,7 +486,9 @@ static void launch_gemm_offs(const GemmSet &set, size_t tiles, const ActView &av
   if constexpr (KW == 1) {
     GemmSet wide = set;
     const size_t wide_tiles = gemm_column_tiles(wide, 4);
-    const GemmTile t = gemm_tile_rule(tiles, wide_tiles, av.mgroups, OFFS);
+    bool wide_ok = !OFFS;
+    for (int i = 0; i < set.count; ++i) wide_ok = wide_ok && !(set.it[i].flags & (GEMM_KOP | GEMM_VOP));
+    const GemmTile t = gemm_tile_rule(tiles, wide_tiles, av.mgroups, wide_ok);
     if constexpr (!OFFS)
       if (t.tn == 4) return launch_gemm_tm<DT, 1, 3, false, 4>(wide, wide_tiles, av, m, s);
     if (t.tm == 3) return launch_gemm_tm<DT, 1, 3, OFFS>(set, tiles, av, m, s);
@@ -515,7 +517,7 @@ static void launch_gemm_dt(const GemmSet &set, size_t tiles, const ActView &av, 
 // with 32-bit byte offsets (buffer loads), so every plane stays below 4 GiB.
 static int run_gemm(const rw_weight *const *w, const float *const *bias, float *const *out, size_t count,
                     const ActView &av, int m, hipStream_t s, const int *flags = nullptr, int8_t *qo = nullptr,
-                    float *ao = nullptr) {
+                    float *ao = nullptr, uint16_t *kv = nullptr) {
   const size_t lim = (size_t)1 << 32;
   if ((size_t)av.mgroups * (size_t)w[0]->nb * 2048 >= lim)
     return fail(RW_EINVAL, "activation [%d, %zu] too large for the GEMM's 32-bit offsets", m, w[0]->k);
@@ -537,6 +539,8 @@ static int run_gemm(const rw_weight *const *w, const float *const *bias, float *
     it.flags = flags ? flags[i] : 0;
     it.qo = qo;
     it.ao = ao;
+    it.kv = kv;
+    it.kv_nblk = av.mgroups;
     it.tile0 = (int)tiles;
     tiles += cdiv(w[i]->ngroups, GEMM_TN);
   }
@@ -1381,7 +1385,7 @@ struct LayerLayout {
   size_t n, f;
   ActLayout act;  // the quantized activation of the widest product (fc2's)
   AttnLayout att;
-  size_t off_act, off_q, off_k, off_v, off_a, off_h, off_att, bytes;
+  size_t off_act, off_q, off_a, off_h, off_att, bytes;
 };
 
 static LayerLayout layer_layout(size_t n, size_t f, size_t t) {
@@ -1393,9 +1397,7 @@ static LayerLayout layer_layout(size_t n, size_t f, size_t t) {
   const size_t row = t * n * 4;
   L.off_act = 0;
   L.off_q = align_up(L.act.bytes, 256);
-  L.off_k = align_up(L.off_q + row, 256);
-  L.off_v = align_up(L.off_k + row, 256);
-  L.off_a = align_up(L.off_v + row, 256);
+  L.off_a = align_up(L.off_q + row, 256);
   L.off_h = align_up(L.off_a + row, 256);
   L.off_att = align_up(L.off_h + std::max(t * f * 4, fused_quant_bytes(t, f)), 256);
   L.bytes = align_up(L.off_att + L.att.bytes, 256);
@@ -1427,7 +1429,8 @@ static int check_layer(const rw_encoder_layer *E, size_t t) {
 static int run_encoder_layer(const rw_encoder_layer *E, float *x, size_t t, void *ws, hipStream_t s) {
   const LayerLayout L = layer_layout(E->q->k, E->fc1->n, t);
   char *b = (char *)ws;
-  float *qb = (float *)(b + L.off_q), *kb = (float *)(b + L.off_k), *vb = (float *)(b + L.off_v);
+  float *qb = (float *)(b + L.off_q);
+  uint16_t *kv = (uint16_t *)(b + L.off_att + L.att.off_kv);
   float *ab = (float *)(b + L.off_a), *hb = (float *)(b + L.off_h);
   const size_t n = L.n, f = L.f;
   const ActLayout Ln = act_layout(t, n), Lf = act_layout(t, f);
@@ -1438,11 +1441,14 @@ static int run_encoder_layer(const rw_encoder_layer *E, float *x, size_t t, void
   {
     const rw_weight *w3[3] = {E->q, E->k, E->v};
     const float *b3[3] = {E->q_b, E->k_b, E->v_b};
-    float *o3[3] = {qb, kb, vb};
-    rc = run_gemm(w3, b3, o3, 3, act_view(Ln, b), m, s);
+    float *o3[3] = {qb, nullptr, nullptr};
+    // k and v leave their products as attention operands
+    const int f3[3] = {0, GEMM_KOP, GEMM_VOP};
+    rc = run_gemm(w3, b3, o3, 3, act_view(Ln, b), m, s, f3, nullptr, nullptr, kv);
     if (rc) return rc;
   }
-  rc = run_attention(qb, n, kb, n, vb, n, t, t, E->n_head, 0, ab, n, L.att, b + L.off_att, s);
+  const AttnPlanes kvp{kv, 0, L.att.tkv_pad};
+  rc = run_attention(qb, n, nullptr, n, nullptr, n, t, t, E->n_head, 0, ab, n, L.att, b + L.off_att, s, &kvp);
   if (rc) return rc;
   rc = launch_quantize(ab, t, n, Ln, b, s);
   if (rc) return rc;
@@ -2218,17 +2224,25 @@ int rw_rocm_decoder_set_audio_dev(rw_decoder *d, const float *enc_out, void *str
   RW_TRY(launch_quantize(enc_out, T, n, AL, b + off_act, s));
   for (int l = 0; l < d->p.n_layer; ++l) {
     const rw_decoder_layer &L = d->layers[l];
-    if (T > (size_t)GEMV_MAX_M && L.ck->dtype == L.cv->dtype && L.ck->k == L.cv->k) {
+    const AttnPlanes cp = d->cross->planes(l);
+    uint16_t *kv = const_cast<uint16_t *>(cp.kv);
+    if (T > (size_t)GEMV_MAX_M) {  // the products write the attention operands
       const rw_weight *w2[2] = {L.ck, L.cv};
       const float *b2[2] = {nullptr, L.cv_b};  // the key has no bias
-      float *o2[2] = {kf, vf};
-      RW_TRY(run_gemm(w2, b2, o2, 2, act_view(AL, b + off_act), (int)T, s));
+      float *o2[2] = {nullptr, nullptr};
+      const int f2[2] = {GEMM_KOP, GEMM_VOP};
+      const ActView av = act_view(AL, b + off_act);
+      if (L.ck->dtype == L.cv->dtype && L.ck->k == L.cv->k) {
+        RW_TRY(run_gemm(w2, b2, o2, 2, av, (int)T, s, f2, nullptr, nullptr, kv));
+      } else {
+        for (int i = 0; i < 2; ++i)
+          RW_TRY(run_gemm(w2 + i, b2 + i, o2 + i, 1, av, (int)T, s, f2 + i, nullptr, nullptr, kv));
+      }
     } else {
       RW_TRY(run_product(L.ck, T, nullptr, kf, b + off_act, s));
       RW_TRY(run_product(L.cv, T, L.cv_b, vf, b + off_act, s));
+      RW_TRY(launch_attn_split(kf, n, vf, n, T, d->p.n_head, kv, cp.tkv_pad / ATT_KVB, s));
     }
-    const AttnPlanes cp = d->cross->planes(l);
-    RW_TRY(launch_attn_split(kf, n, vf, n, T, d->p.n_head, const_cast<uint16_t *>(cp.kv), cp.tkv_pad / ATT_KVB, s));
   }
   d->audio = true;
   d->n_past = 0;

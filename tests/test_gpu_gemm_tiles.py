@@ -1,0 +1,63 @@
+"""Edges of the GEMM's tile choice and of the epilogues that write attention
+operands (run_gemm's rules in rw_rocm.hip, GEMM_KOP / GEMM_VOP in
+rw_kernels.hpp)."""
+import numpy as np
+import pytest
+
+import oracle as O
+from oracle.decoder import Decoder as OD
+from oracle.encoder import encoder_layer
+from rusty_whisper_amd import _abi as A
+from _decoder_params import decoder_params
+from test_gpu_decoder import device_decoder, rel, step, torch  # noqa: F401
+from test_gpu_encoder_layer import build, rel_row
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [2, 7, 8])
+@pytest.mark.parametrize("m", [3833, 3904, 2900])
+def test_tile_choice_keeps_rows(torch, dtype, m):  # noqa: F811
+    """3150 columns at k = 64 run 96 x 128 tiles at 3833 rows (one round), 128 x
+    64 at 3904, 96 x 64 at 2900, and 64-row tiles at 60; the same rows are the
+    same bits in each, and within the matmul's 1e-3 of the oracle."""
+    n, k = 3150, 64
+    rng = np.random.default_rng(m + dtype)
+    raw = O.quantize(dtype, (rng.standard_normal((n, k)) * 0.05).astype(np.float32))
+    a, bias = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal(n).astype(np.float32)
+    w = A.DeviceWeight(dtype, n, k, raw)
+    full = w.matmul(a, bias)
+    rows = np.r_[0:30, m - 30:m]
+    assert np.array_equal(w.matmul(a[rows], bias).view(np.uint32), full[rows].view(np.uint32))
+    ref = O.matmul_emul(a[rows], dtype, raw, n, bias=bias).astype(np.float64)
+    assert np.max(np.abs(full[rows] - ref) / np.linalg.norm(ref, axis=1, keepdims=True)) <= 1e-3
+
+
+@pytest.mark.parametrize("t,n", [(9, 64), (31, 128), (32, 128), (33, 192), (97, 1024), (640, 1024)], ids=str)
+def test_encoder_layer_attention_operands(torch, t, n):  # noqa: F811
+    """Rows around the 32-row blocks, one head up, k-split and single-wavefront
+    launches: the encoder layer's bars (test_gpu_encoder_layer.py)."""
+    p, dev = build(torch, n, 2 * n, 6, seed=t + n)
+    x = np.random.default_rng(t).standard_normal((t, n)).astype(np.float32)
+    xd = torch.from_numpy(x).to("cuda:0")
+    A.EncoderLayer(n // 64, **dev).run(xd, t)
+    torch.cuda.synchronize()
+    got, ref = xd.cpu().numpy(), encoder_layer(x, p, n // 64)
+    assert rel_row(got, ref) <= 2e-3
+    assert rel_row(got - x, ref - x) <= 3e-3
+
+
+@pytest.mark.parametrize("mixed", [False, True])
+@pytest.mark.parametrize("n_audio", [8, 9, 33, 64])
+def test_cross_attention_operands(torch, n_audio, mixed):  # noqa: F811
+    """The window's K and V from 8 rows (f32 rows, then split) and more (written
+    by the products, one launch or one each), against the decoder's 4e-3 bar."""
+    n, heads = 192, 3
+    p = decoder_params(n=n, f=2 * n, n_layer=1, n_vocab=100, n_ctx=16, dtype=8, seed=n_audio,
+                       dtypes={"cv": 7} if mixed else None)
+    enc = np.random.default_rng(n_audio).standard_normal((n_audio, n)).astype(np.float32)
+    d = device_decoder(torch, p, heads, n_audio)
+    d.set_audio(torch.from_numpy(enc).to("cuda:0"))
+    o = OD(p, heads, enc)
+    for toks in ([1, 2, 3], [4], list(range(9))):
+        assert rel(step(torch, d, toks, n), o.forward_hidden(toks)) <= 4e-3
