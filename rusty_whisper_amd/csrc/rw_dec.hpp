@@ -12,33 +12,40 @@ namespace rw {
 
 #if defined(__HIPCC__)
 
+// the token ids of a step of at most EMBED_IDS rows, passed by value: a copy of
+// 4 to 32 bytes to the device was a launch of its own, 4 us and the gaps beside
+// it
+constexpr int EMBED_IDS = 8;
+struct EmbedIds {
+  int id[EMBED_IDS];
+};
+
 // x[i] = token_embedding.row_f32(tok[i]) + positional[n_past + i * pos_step]
 // (src/decoder.rs:122-135): the quantized row dequantized as d * q + m (two
 // roundings), then the position added.  pos_step is 1 for a prompt's
-// consecutive tokens and 0 for one token of each of several beams.  One
-// thread per (token, block).
+// consecutive tokens and 0 for one token of each of several beams.  One thread
+// per element, blockIdx.y the token; tok NULL: the ids come in `ids`.
 template <int DT>
-__global__ __launch_bounds__(256) void k_embed(WeightView w, const int *__restrict__ tok, int n_tok,
+__global__ __launch_bounds__(256) void k_embed(WeightView w, const int *__restrict__ tok, EmbedIds ids,
                                                const float *__restrict__ pos, int n_past, int pos_step,
                                                float *__restrict__ x) {
-  const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (size_t)n_tok * w.nb) return;
-  const int bl = (int)(t % w.nb), i = (int)(t / w.nb);
-  const int j = tok[i];
+  const size_t n = (size_t)w.nb * QK, c = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (c >= n) return;
+  const int i = blockIdx.y, bl = (int)(c / QK);
+  const int j = tok ? tok[i] : ids.id[i & (EMBED_IDS - 1)];
   const int g = j / RG, r = j % RG;
   const size_t si = sc_index(w, g, bl, r);
   const float d = h2f_exact(w.d[si]);
   const float m = has_min(DT) ? h2f_exact(w.m[si]) : 0.0f;
-  const size_t n = (size_t)w.nb * QK;
-  float *o = x + (size_t)i * n + (size_t)bl * QK;
-  const float *p = pos + (size_t)(n_past + i * pos_step) * n + (size_t)bl * QK;
-  for (int e = 0; e < QK; ++e) o[e] = __fadd_rn(__fadd_rn(__fmul_rn(d, (float)weight_q<DT>(w, g, bl, r, e)), m), p[e]);
+  x[(size_t)i * n + c] = __fadd_rn(__fadd_rn(__fmul_rn(d, (float)weight_q<DT>(w, g, bl, r, (int)(c % QK))), m),
+                                   pos[(size_t)(n_past + i * pos_step) * n + c]);
 }
 
 // y = layernorm(x) row by row (src/tensor.rs:274-287): mean, mean of squared
 // deviations, inv = 1 / sqrt(var + 1e-5), (x - mean) * inv * w + b; the sums
 // in tree order.  One workgroup per row.  With r != NULL the residual add
 // comes first: x += r (stored back), then y = layernorm(x).
+constexpr int LN_REG = 8;
 __global__ __launch_bounds__(256) void k_layernorm(float *__restrict__ x, int n, const float *__restrict__ w,
                                                    const float *__restrict__ b, float *__restrict__ y,
                                                    const float *__restrict__ r) {
@@ -57,6 +64,31 @@ __global__ __launch_bounds__(256) void k_layernorm(float *__restrict__ x, int n,
     __syncthreads();
     return (part[slot][0] + part[slot][1]) + (part[slot][2] + part[slot][3]);
   };
+  float *yr = y + (size_t)row * n;
+  // rows of at most 256 LN_REG values stay in registers (one read of the row;
+  // the same sums in the same order)
+  if (n <= 256 * LN_REG) {
+    float v[LN_REG], s = 0.0f;
+#pragma unroll
+    for (int u = 0; u < LN_REG; ++u) v[u] = t + 256 * u < n ? xr[t + 256 * u] : 0.0f;
+#pragma unroll
+    for (int u = 0; u < LN_REG; ++u)
+      if (t + 256 * u < n) s += v[u];
+    const float mean = __fdiv_rn(reduce(s, 0), (float)n);
+    s = 0.0f;
+#pragma unroll
+    for (int u = 0; u < LN_REG; ++u)
+      if (t + 256 * u < n) {
+        const float d = v[u] - mean;
+        s += d * d;
+      }
+    const float var = __fdiv_rn(reduce(s, 1), (float)n);
+    const float inv = __fdiv_rn(1.0f, __fsqrt_rn(var + 1e-5f));
+#pragma unroll
+    for (int u = 0; u < LN_REG; ++u)
+      if (t + 256 * u < n) yr[t + 256 * u] = (v[u] - mean) * inv * w[t + 256 * u] + b[t + 256 * u];
+    return;
+  }
   float s = 0.0f;
   for (int c = t; c < n; c += 256) s += xr[c];
   const float mean = __fdiv_rn(reduce(s, 0), (float)n);
@@ -67,7 +99,6 @@ __global__ __launch_bounds__(256) void k_layernorm(float *__restrict__ x, int n,
   }
   const float var = __fdiv_rn(reduce(s, 1), (float)n);
   const float inv = __fdiv_rn(1.0f, __fsqrt_rn(var + 1e-5f));
-  float *yr = y + (size_t)row * n;
   for (int c = t; c < n; c += 256) yr[c] = (xr[c] - mean) * inv * w[c] + b[c];
 }
 

@@ -1295,20 +1295,26 @@ static int launch_layernorm(float *x, size_t rows, size_t n, const float *w, con
 // One forward pass: n_tok tokens of one decoder (nb = 1, beams = false), or
 // one token for each of nb beams (forks sharing the cross K/V at one n_past,
 // n_tok = nb, beams = true).
-static int decoder_forward(rw_decoder *const *dec, size_t nb, bool beams, size_t n_tok, float *hidden, char *b,
-                           const DecScratch &S, hipStream_t s) {
+static int decoder_forward(rw_decoder *const *dec, size_t nb, bool beams, const uint32_t *tokens, size_t n_tok,
+                           float *hidden, char *b, const DecScratch &S, hipStream_t s) {
   rw_decoder *d = dec[0];
   const size_t n = d->n;
-  const int *tok = (const int *)(b + S.off_tok);
+  // (at most EMBED_IDS token ids by value, a longer prompt's copied first)
+  const int *tok = n_tok > (size_t)EMBED_IDS ? (const int *)(b + S.off_tok) : nullptr;
+  EmbedIds ids{};
+  if (tok)
+    HIP_TRY(hipMemcpyAsync(b + S.off_tok, tokens, n_tok * 4, hipMemcpyHostToDevice, s));
+  else
+    for (size_t i = 0; i < n_tok; ++i) ids.id[i] = (int)tokens[i];
   float *x = (float *)(b + S.off_x), *cur = (float *)(b + S.off_cur), *q = (float *)(b + S.off_q);
   float *att = (float *)(b + S.off_a), *h = (float *)(b + S.off_h);
   float *kn = (float *)(b + S.off_kn), *vn = (float *)(b + S.off_vn);
   void *act = b + S.off_act, *aws = b + S.off_att;
   const rw_weight *E = d->p.token_embedding;
-  const size_t items = n_tok * (size_t)E->nb;
+  const dim3 egrid((unsigned)cdiv(n, 256), (unsigned)n_tok);
 #define RW_EMB(DT)                                                                                           \
-  hipLaunchKernelGGL(k_embed<DT>, dim3((unsigned)cdiv(items, 256)), dim3(256), 0, s, E->view, tok, (int)n_tok, \
-                     d->p.positional, (int)d->n_past, beams ? 0 : 1, x)
+  hipLaunchKernelGGL(k_embed<DT>, egrid, dim3(256), 0, s, E->view, tok, ids, d->p.positional, (int)d->n_past, \
+                     beams ? 0 : 1, x)
   switch (E->dtype) {
     case RW_Q4_0: RW_EMB(RW_Q4_0); break;
     case RW_Q4_1: RW_EMB(RW_Q4_1); break;
@@ -2312,8 +2318,7 @@ int rw_rocm_decoder_forward_hidden_dev(rw_decoder *d, const uint32_t *tokens, si
   if (rc) return rc;
   char *b = (char *)d->scratch;
   hipStream_t s = (hipStream_t)stream;
-  HIP_TRY(hipMemcpyAsync(b + S.off_tok, tokens, n_tok * 4, hipMemcpyHostToDevice, s));
-  rc = decoder_forward(&d, 1, false, n_tok, hidden, b, S, s);
+  rc = decoder_forward(&d, 1, false, tokens, n_tok, hidden, b, S, s);
   if (rc) return rc;
   d->n_past += n_tok;
   return RW_OK;
@@ -2347,8 +2352,7 @@ int rw_rocm_decoder_forward_beams_dev(rw_decoder *const *beams, size_t n_beams, 
   if (rc) return rc;
   char *b = (char *)d->scratch;
   hipStream_t s = (hipStream_t)stream;
-  HIP_TRY(hipMemcpyAsync(b + S.off_tok, tokens, n_beams * 4, hipMemcpyHostToDevice, s));
-  rc = decoder_forward(beams, n_beams, true, n_beams, hidden, b, S, s);
+  rc = decoder_forward(beams, n_beams, true, tokens, n_beams, hidden, b, S, s);
   if (rc) return rc;
   for (size_t i = 0; i < n_beams; ++i) beams[i]->n_past += 1;
   return RW_OK;
