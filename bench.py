@@ -291,7 +291,7 @@ def time_decode(A, torch, D, steps: int, warmup: int, stream):
 def time_attention(A, torch, stream, steps: int, warmup: int, t: int = 1500, n_state: int = 1280, n_head: int = 20):
     """One encoder layer's self-attention (large-v3: 20 heads of 64 over 1500
     positions) through rw_rocm_attention_dev on resident q, k, v: ms per
-    call (the three split launches and k_attn) and the algorithmic flops
+    call (the split launch and k_attn_tile) and the algorithmic flops
     (2 t^2 dh per head for Q K^T, the same for P V)."""
     g = torch.Generator(device="cuda:0")
     g.manual_seed(11)
@@ -1094,7 +1094,7 @@ def main() -> int:
             "us_per_layer": round(ams * 1e3, 2),
             "flops": aflops,
             "TFLOP_per_s": round(atf, 2),
-            "launch": "rw_rocm_attention_dev: one split launch (q, k, v to f16 hi/lo planes) and one k_attn",
+            "launch": "rw_rocm_attention_dev: one split launch (k, v to f16 hi/lo operand blocks) and one k_attn_tile",
             "note": "algorithmic flops 4*t^2*64 per head; each product runs as three f16 MFMA products",
         }
 
