@@ -46,6 +46,7 @@ constexpr int ATT_QB = 64;   // query rows a workspace's rows are padded to
 constexpr int ATT_NK = 4;    // wavefronts of a k_attn_tile workgroup
 constexpr int ATT_STEP_MAX = 8;   // query rows of a k_attn call at most
 constexpr int ATT_ROWS_MAX = 64;  // query rows of a call that splits K and V as it loads them, at most
+constexpr int ATT_TILE_ROWS_BLK = 20;  // kv blocks of a k_attn_tile call that splits K and V itself, at most
 #ifndef ATT_MAX_SPLIT_N
 #define ATT_MAX_SPLIT_N 32
 #endif
@@ -562,8 +563,8 @@ __global__ __launch_bounds__(64 * ATT_NK, 2) void k_attn_tile(int t_q, int t_kv,
   }
 }
 
-// Calls of at most 8 query rows.  Workgroup (blockIdx.x, blockIdx.y) = (32
-// query rows, head); wavefront w takes kv
+// Calls of at most 8 query rows, or of at most 64 against many keys of their own
+// (ROWS).  Workgroup (blockIdx.x, blockIdx.y) = (32 query rows, head); wavefront w takes kv
 // blocks w, w + 2, ...; a causal query row i (at absolute position t_kv - t_q
 // + i) sees kv rows up to its position.
 //

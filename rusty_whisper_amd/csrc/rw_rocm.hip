@@ -1166,7 +1166,12 @@ static int run_attention(const float *q, size_t ldq, const float *k, size_t ldk,
   if (kv_split) P.kv = kv_split->kv, P.tkv_pad = kv_split->tkv_pad;
   const int nblk = P.tkv_pad / ATT_KVB;
   const bool rows = !kv_split && t_q <= (size_t)ATT_ROWS_MAX;
-  if (t_q > (size_t)ATT_STEP_MAX) {
+  // 9 to 64 query rows against many keys of their own: k_attn's kv split over
+  // workgroups and its merge (20 rows against 1500, 20 heads: 11.7 us, where
+  // k_attn_tile's chain of 12 blocks per wavefront takes 21.9; against 448 keys
+  // 11.8 and 10.2)
+  const bool long_rows = rows && cdiv(t_kv, ATT_KVB) > (size_t)ATT_TILE_ROWS_BLK;
+  if (t_q > (size_t)ATT_STEP_MAX && !long_rows) {
     if (!kv_split && !rows)
       RW_TRY(launch_attn_split(k, ldk, v, ldv, t_kv, n_head, (uint16_t *)(b + L.off_kv), nblk, s));
     // 64 query rows per workgroup where those fill 3/4 of the 512 workgroup
@@ -1187,13 +1192,13 @@ static int run_attention(const float *q, size_t ldq, const float *k, size_t ldk,
   // with the kv length, so this one fits the layout's part buffer)
   const int nsplit = std::min(L.nsplit, attn_nsplit((size_t)n_head, cdiv(t_kv, ATT_KVB)));
   float *part = nsplit > 1 ? (float *)(b + L.off_part) : nullptr;
-  const dim3 grid(1u, (unsigned)n_head, (unsigned)nsplit);
+  const dim3 grid((unsigned)cdiv(t_q, 32), (unsigned)n_head, (unsigned)nsplit);
   const int gw = (causal ? 1 : 0) | nsplit << 1 | n_head << 8;  // k_attn's packed grid
   if (rows)
-    hipLaunchKernelGGL((k_attn<true>), grid, dim3(128), 0, s, (int)t_q, (int)t_kv, gw, 1, q, (int)ldq, k, (int)ldk, v,
+    hipLaunchKernelGGL((k_attn<true>), grid, dim3(128), 0, s, (int)t_q, (int)t_kv, gw, (int)grid.x, q, (int)ldq, k, (int)ldk, v,
                        (int)ldv, out, (int)ldo, part, P, nullptr, 0, BeamCaches{});
   else
-    hipLaunchKernelGGL((k_attn<false>), grid, dim3(128), 0, s, (int)t_q, (int)t_kv, gw, 1, q, (int)ldq, nullptr, 0,
+    hipLaunchKernelGGL((k_attn<false>), grid, dim3(128), 0, s, (int)t_q, (int)t_kv, gw, (int)grid.x, q, (int)ldq, nullptr, 0,
                        nullptr, 0, out, (int)ldo, part, P, nullptr, 0, BeamCaches{});
   LAUNCH_TRY("k_attn");
   if (part) {
