@@ -18,7 +18,8 @@
 // 22 of f32's 24 significant bits and the dropped lo*lo term is below 2^-22
 // of the product, so outputs stay within about 1e-6 (relative to the row) of
 // the exact result, like the reference's f32 arithmetic.  Probabilities
-// enter scaled by 2^8 or more (ATT_PS) so that small ones keep their f16 bits.
+// enter scaled to 2^12 or more at the row's maximum (ATT_PS), so that small
+// ones keep their f16 bits: a step of 2^-24 is 2^-36 of the largest.
 // Inputs must stay below f16's 65504 in magnitude (whisper's projections are
 // far below it); inputs below about 1e-3 lose a few bits to f16 subnormal
 // residuals.  The softmax is online (running reference exponent and sum per
@@ -265,14 +266,18 @@ __device__ inline void att_split_v(const AttVRaw &x, AttV &o) {
 
 // The softmax's running state of one query (a lane pair (n, n + 32) holds one):
 // cm, a reference exponent, and lsum, this lane's sum of p = 2^(log2(e) s -
-// cm).  cm is set ATT_PS = 8 below log2(e) times the largest score seen, and
-// moved only when a score passes it by more than ATT_PS + ATT_SLACK (p <= 2^15
-// fits f16): then the output and the sum are rescaled.  Any cm gives the same
-// quotient, so its own rounding cancels; p = 2^8 .. 2^15 at the row's maximum
-// keeps small probabilities' f16 bits (hi + lo hold 2^-24 absolute).  Rescaling
-// at every new maximum moved some query of a tile in nearly every block (a
-// wavefront sees 12 of them at t = 1500).
-constexpr float ATT_PS = 8.0f, ATT_SLACK = 7.0f, ATT_NONE = -1e30f;  // ATT_NONE: no score seen yet
+// cm).  cm is set ATT_PS = 12 below log2(e) times the largest score seen, and
+// moved only when a score passes it by more than ATT_PS + ATT_SLACK (p <=
+// 2^15.9 fits f16): then the output and the sum are rescaled.  Any cm gives the
+// same quotient, so its own rounding cancels; p >= 2^12 at the row's maximum is
+// what keeps small probabilities' f16 bits (hi + lo hold 2^-24 absolute, 2^-36
+// of the maximum): where a row's mass is on one key of little value, its output
+// is made of probabilities far below the maximum, and with p = 2^8 there its
+// error was 16 times larger (a gap of 2^20: up to 4e-5 of the row).
+// Rescaling at every new maximum moved some query of a tile in nearly every
+// block (a wavefront sees 12 of them at t = 1500); with 3.9 bits of slack it is
+// a few of them (20 heads, t = 1500: 43.6 us, 42.9 with 7 bits).
+constexpr float ATT_PS = 12.0f, ATT_SLACK = 3.9f, ATT_NONE = -1e30f;  // ATT_NONE: no score seen yet
 
 // the largest score of the query's 32 kv rows (s: lane (h, n) holds query n's
 // rows 8 (i / 4) + 4 h + i % 4), as the cm it asks for

@@ -58,3 +58,29 @@ def test_moving_maxima(t_q, step):
     q[:, ::64] = 8.0  # score = the key's first value
     k[:, ::64] = (step * np.arange(t_kv, dtype=np.float32))[:, None]
     assert err(A.attention(q, k, v, heads, False), q, k, v, heads, False) <= 1e-5
+
+
+@pytest.mark.parametrize("t_q", [8, 40, 100, 1030])
+@pytest.mark.parametrize("gap", [12, 16, 18, 20])
+def test_mass_on_a_key_without_value(t_q, gap):
+    """Rows whose probability sits on keys of value 0 (an attention sink), so
+    that the output is made of the other keys' probabilities, 2^-gap of the
+    row's largest.  P enters the products as f16 pairs of 2^12 or more at the
+    maximum, in steps of 2^-24: an error of 2^-37 of the maximum per key,
+    2^(gap - 37) of the others, and half of that over a row's norm leaves room
+    for the sums (beside the 1e-6 of any row)."""
+    heads, t_kv = 24, 320
+    rng = np.random.default_rng(gap)
+    q = np.zeros((t_q, 64 * heads), np.float32)
+    k = np.zeros((t_kv, 64 * heads), np.float32)
+    v = rng.standard_normal((t_kv, 64 * heads)).astype(np.float32)
+    q[:, ::64] = 8.0  # score = the key's first value, exact in the f16 pairs
+    k[:, ::64] = np.round(rng.uniform(-0.5, 0.5, (t_kv, heads)) * 1024) / 1024
+    sinks = np.arange(0, 128, 32)  # one in each wavefront's first block
+    k[sinks, ::64] = np.round(gap * np.log(2) * 256) / 256
+    v[sinks] = 0.0
+    got = A.attention(q, k, v, heads, False).astype(np.float64)
+    ref = mha(q, k, v, heads, False, dtype=np.float64)
+    rows = lambda x: x.reshape(t_q * heads, 64)  # noqa: E731  a head's row
+    e = np.max(np.abs(rows(got - ref)), axis=1) / np.linalg.norm(rows(ref), axis=1)
+    assert e.max() <= 1e-6 + 0.5 * 2.0 ** (gap - 37), e.max()
