@@ -265,38 +265,45 @@ __device__ inline void att_split_v(const AttVRaw &x, AttV &o) {
 }
 
 // The softmax's running state of one query (a lane pair (n, n + 32) holds one):
-// cm, a reference exponent, and lsum, this lane's sum of p = 2^(log2(e) s -
-// cm).  cm is set ATT_PS = 12 below log2(e) times the largest score seen, and
-// moved only when a score passes it by more than ATT_PS + ATT_SLACK (p <=
-// 2^15.9 fits f16): then the output and the sum are rescaled.  Any cm gives the
-// same quotient, so its own rounding cancels; p >= 2^12 at the row's maximum is
-// what keeps small probabilities' f16 bits (hi + lo hold 2^-24 absolute, 2^-36
-// of the maximum): where a row's mass is on one key of little value, its output
-// is made of probabilities far below the maximum, and with p = 2^8 there its
-// error was 16 times larger (a gap of 2^20: up to 4e-5 of the row).
-// Rescaling at every new maximum moved some query of a tile in nearly every
-// block (a wavefront sees 12 of them at t = 1500); with 3.9 bits of slack it is
-// a few of them (20 heads, t = 1500: 43.6 us, 42.9 with 7 bits).
-constexpr float ATT_PS = 12.0f, ATT_SLACK = 3.9f, ATT_NONE = -1e30f;  // ATT_NONE: no score seen yet
+// m, a reference score, and lsum, this lane's sum of p = 2^(log2(e) (s - m) +
+// ATT_PS).  m is the largest score seen when it was set, and moved only when a
+// score passes it by more than ATT_SLACK (3.9 bits: p <= 2^15.9 fits f16): then
+// the output and the sum are rescaled.  Any m gives the same quotient; p >= 2^12
+// at the row's maximum is what keeps small probabilities' f16 bits (hi + lo hold
+// 2^-24 absolute, 2^-36 of the maximum): where a row's mass is on one key of
+// little value, its output is made of probabilities far below the maximum, and
+// with p = 2^8 there its error was 16 times larger (a gap of 2^20: up to 4e-5 of
+// the row).  s - m comes before the factor, as a score's difference from one near
+// it is exact: with log2(e) m rounded on its own, scores past 2^26 (|q|, |k| in
+// the thousands) left every p at infinity or 0 (one instruction less per score,
+// 43.6 against 44.0 us at 20 heads and t = 1500).  Rescaling at every new maximum
+// moved some query of a tile in nearly every block (a wavefront sees 12 of them
+// at t = 1500); with 3.9 bits of slack it is a few of them.
+constexpr float ATT_PS = 12.0f, ATT_SLACK = 3.9f / ATT_LOG2E;
+constexpr float ATT_NONE = -1e30f;  // no score seen yet
 
 // the largest score of the query's 32 kv rows (s: lane (h, n) holds query n's
-// rows 8 (i / 4) + 4 h + i % 4), as the cm it asks for
+// rows 8 (i / 4) + 4 h + i % 4)
 __device__ inline float att_block_max(const att_v16f &s) {
   float mx = fmaxf(s[0], s[1]);
 #pragma unroll
   for (int i = 2; i < 16; i += 2) mx = fmaxf(fmaxf(mx, s[i]), s[i + 1]);
   const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
-  return __builtin_fmaf(fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1])), ATT_LOG2E, -ATT_PS);
+  return fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
 }
-// does some query of the wavefront need a new cm?
-__device__ inline bool att_moved(float cm, float cb) { return __builtin_amdgcn_ballot_w64(cb > cm + ATT_SLACK) != 0; }
-__device__ inline void att_rescale(float cb, float &cm, float &lsum, att_v16f (&o)[2]) {
-  const float cnew = cb > cm + ATT_SLACK ? cb : cm;
-  const float alpha = __builtin_amdgcn_exp2f(cm - cnew);
+// does some query of the wavefront need a new m?  (the difference, which is exact
+// between close scores: m + ATT_SLACK would round to more than the slack where
+// scores are large)
+__device__ inline bool att_moved(float m, float mx) {
+  return __builtin_amdgcn_ballot_w64(mx - m > ATT_SLACK) != 0;
+}
+__device__ inline void att_rescale(float mx, float &m, float &lsum, att_v16f (&o)[2]) {
+  const float mnew = mx - m > ATT_SLACK ? mx : m;
+  const float alpha = __builtin_amdgcn_exp2f((m - mnew) * ATT_LOG2E);
   lsum *= alpha;
   o[0] *= alpha;
   o[1] *= alpha;
-  cm = cnew;
+  m = mnew;
 }
 // p - hi, one mixed-precision FMA each (the compiler converts and subtracts)
 __device__ inline att_v2f att_resid(att_v2f p, att_v2h hi) {
@@ -306,13 +313,13 @@ __device__ inline att_v2f att_resid(att_v2f p, att_v2h hi) {
   asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r.y) : "v"(hb), "v"(p.y));
   return r;
 }
-// scores to the P^T operands, one FMA and one exp2 each; their sum to lsum
-__device__ inline void att_probs(const att_v16f &s, float cm, float &lsum, att_v8h (&ph)[2], att_v8h (&pl)[2]) {
+// scores to the P^T operands; their sum to lsum
+__device__ inline void att_probs(const att_v16f &s, float m, float &lsum, att_v8h (&ph)[2], att_v8h (&pl)[2]) {
   float s0 = 0.0f, s1 = 0.0f;
 #pragma unroll
   for (int i = 0; i < 16; i += 2) {
-    const att_v2f p = {__builtin_amdgcn_exp2f(__builtin_fmaf(s[i], ATT_LOG2E, -cm)),
-                       __builtin_amdgcn_exp2f(__builtin_fmaf(s[i + 1], ATT_LOG2E, -cm))};
+    const att_v2f p = {__builtin_amdgcn_exp2f(__builtin_fmaf(s[i] - m, ATT_LOG2E, ATT_PS)),
+                       __builtin_amdgcn_exp2f(__builtin_fmaf(s[i + 1] - m, ATT_LOG2E, ATT_PS))};
     s0 += p.x;
     s1 += p.y;
     const att_v2h hi = __builtin_convertvector(p, att_v2h);  // one packed conversion
@@ -441,17 +448,17 @@ __global__ __launch_bounds__(64 * ATT_NK, 2) void k_attn_tile(int t_q, int t_kv,
   }
 
   att_v16f o[QT][2];  // O^T
-  float cm[QT], lsum[QT];
+  float m[QT], lsum[QT];
 #pragma unroll
   for (int qt = 0; qt < QT; ++qt) {
     o[qt][0] = (att_v16f){};
     o[qt][1] = (att_v16f){};
-    cm[qt] = ATT_NONE;
+    m[qt] = ATT_NONE;
     lsum[qt] = 0.0f;
   }
   int b = wv;
   att_v16f s[QT];
-  float cb[QT];
+  float mx[QT];
   // block b's scores and maxima, K's next block requested behind them
   auto scores = [&]() __attribute__((always_inline)) {
     // (an offset the compiler cannot see through: it would keep all of q's
@@ -478,7 +485,7 @@ __global__ __launch_bounds__(64 * ATT_NK, 2) void k_attn_tile(int t_q, int t_kv,
       const int tq0 = q0 + qt * 32;
       if ((b + 1) * ATT_KVB > t_kv || (causal && (b + 1) * ATT_KVB - 1 > off + tq0))
         att_mask(s[qt], b, h, t_kv, causal, off + tq0 + n);
-      cb[qt] = att_block_max(s[qt]);
+      mx[qt] = att_block_max(s[qt]);
     }
   };
   // Two loops, so that the common path has no rescale to merge with: beside
@@ -489,14 +496,14 @@ __global__ __launch_bounds__(64 * ATT_NK, 2) void k_attn_tile(int t_q, int t_kv,
     scores();
     for (;;) {
 #pragma unroll
-      for (int qt = 0; qt < QT; ++qt) att_rescale(cb[qt], cm[qt], lsum[qt], o[qt]);
+      for (int qt = 0; qt < QT; ++qt) att_rescale(mx[qt], m[qt], lsum[qt], o[qt]);
       bool moved;
       do {
         if constexpr (ROWS) att_split_v(vr, vv);
 #pragma unroll
         for (int qt = 0; qt < QT; ++qt) {
           att_v8h ph[2], pl[2];
-          att_probs(s[qt], cm[qt], lsum[qt], ph, pl);
+          att_probs(s[qt], m[qt], lsum[qt], ph, pl);
 #pragma unroll
           for (int k = 0; k < 2; ++k)
 #pragma unroll
@@ -508,7 +515,7 @@ __global__ __launch_bounds__(64 * ATT_NK, 2) void k_attn_tile(int t_q, int t_kv,
         scores();
         moved = false;
 #pragma unroll
-        for (int qt = 0; qt < QT; ++qt) moved = moved || att_moved(cm[qt], cb[qt]);
+        for (int qt = 0; qt < QT; ++qt) moved = moved || att_moved(m[qt], mx[qt]);
       } while (!moved);
       if (b >= nblk) break;
     }
@@ -521,7 +528,7 @@ __global__ __launch_bounds__(64 * ATT_NK, 2) void k_attn_tile(int t_q, int t_kv,
     const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(lsum[qt]), __float_as_uint(lsum[qt]), false, false);
     const float lt = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
     if (h == 0) {
-      xm[wv][qt * 32 + n] = cm[qt];
+      xm[wv][qt * 32 + n] = m[qt];
       xl[wv][qt * 32 + n] = lt;
     }
   }
@@ -534,10 +541,10 @@ __global__ __launch_bounds__(64 * ATT_NK, 2) void k_attn_tile(int t_q, int t_kv,
     if (wv == 0 && h == 0) {
       float den = 0.0f;
 #pragma unroll
-      for (int w = 0; w < NK; ++w) den += xl[w][qt * 32 + n] * __builtin_amdgcn_exp2f(xm[w][qt * 32 + n] - mu);
+      for (int w = 0; w < NK; ++w) den += xl[w][qt * 32 + n] * __builtin_amdgcn_exp2f((xm[w][qt * 32 + n] - mu) * ATT_LOG2E);
       xinv[qt * 32 + n] = 1.0f / den;
     }
-    const float sc = __builtin_amdgcn_exp2f(cm[qt] - mu);
+    const float sc = __builtin_amdgcn_exp2f((m[qt] - mu) * ATT_LOG2E);
     o[qt][0] *= sc;
     o[qt][1] *= sc;
   }

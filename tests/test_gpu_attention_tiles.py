@@ -84,3 +84,27 @@ def test_mass_on_a_key_without_value(t_q, gap):
     rows = lambda x: x.reshape(t_q * heads, 64)  # noqa: E731  a head's row
     e = np.max(np.abs(rows(got - ref)), axis=1) / np.linalg.norm(rows(ref), axis=1)
     assert e.max() <= 1e-6 + 0.5 * 2.0 ** (gap - 37), e.max()
+
+
+@pytest.mark.parametrize("t_q", [8, 40, 100, 1030])
+@pytest.mark.parametrize("scale", [2048.0, 16384.0, 32768.0])
+def test_scores_of_large_operands(t_q, scale):
+    """q and k of +-scale (below the stated 65504): scores of up to 64 scale^2 / 8
+    (8.6e9 at 32768), far beyond where log2(e) times one is known to a bit.  Every
+    product and sum is exact, and a key that does not share the row's largest
+    score is at least scale^2 / 4 below it, so each row is the mean of its best
+    keys' values."""
+    heads, t_kv = 24, 320
+    rng = np.random.default_rng(int(scale))
+    sign = lambda t: (rng.integers(0, 2, (t, 64 * heads)) * 2 - 1).astype(np.float32)  # noqa: E731
+    q, k = sign(t_q) * np.float32(scale), sign(t_kv) * np.float32(scale)
+    k[5::7] = k[:1]  # ties over blocks of every wavefront
+    k[40:44, :] = q[:4]
+    v = rng.standard_normal((t_kv, 64 * heads)).astype(np.float32)
+    got = A.attention(q, k, v, heads, False)
+    for hd in range(heads):
+        c = slice(64 * hd, 64 * hd + 64)
+        s = q[:, c].astype(np.float64) @ k[:, c].astype(np.float64).T
+        best = s == s.max(axis=1, keepdims=True)
+        ref = best @ v[:, c].astype(np.float64) / best.sum(axis=1, keepdims=True)
+        assert np.max(np.max(np.abs(got[:, c] - ref), axis=1) / np.linalg.norm(ref, axis=1)) <= 1e-6, hd
