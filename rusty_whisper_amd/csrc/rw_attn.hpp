@@ -10,8 +10,9 @@
 //   k_attn_tile    calls of more than 8 query rows: one workgroup per (32 or
 //        64 query rows, head), whose 4 wavefronts split the kv blocks
 //        between them and meet in LDS at the end
-//   k_attn    calls of at most 8 query rows (a decoding step): one workgroup of
-//        two wavefronts per (head[, kv run])
+//   k_attn    calls of at most 8 query rows (a decoding step), or of at most 64
+//        against many keys: one workgroup of two wavefronts per (32 query rows,
+//        head[, kv run]); k_attn_combine merges the runs
 //
 // Precision.  Every product runs on v_mfma_f32_32x32x16_f16 as three f16
 // products, hi*hi + hi*lo + lo*hi, accumulated in f32: each operand keeps
@@ -35,6 +36,7 @@
 // 4h..4h+3 and 8+4h..8+4h+3 of each 16, and the v^T operands hold each
 // 16-block of kv positions in that order (attn_vpos).
 #pragma once
+#include <stddef.h>
 #include <stdint.h>
 
 #include "rw_layout.hpp"
@@ -47,12 +49,70 @@ constexpr int ATT_QB = 64;   // query rows a workspace's rows are padded to
 constexpr int ATT_NK = 4;    // wavefronts of a k_attn_tile workgroup
 constexpr int ATT_STEP_MAX = 8;   // query rows of a k_attn call at most
 constexpr int ATT_ROWS_MAX = 64;  // query rows of a call that splits K and V as it loads them, at most
-constexpr int ATT_TILE_ROWS_BLK = 20;  // kv blocks of a k_attn_tile call that splits K and V itself, at most
 #ifndef ATT_MAX_SPLIT_N
 #define ATT_MAX_SPLIT_N 32
 #endif
 constexpr int ATT_MAX_SPLIT = ATT_MAX_SPLIT_N;  // kv runs of one (query block, head) at most
 static_assert(ATT_MAX_SPLIT < 128, "k_attn packs the run count into 7 bits");
+
+// few (query block, head) workgroups -- a decoding step: split the kv
+// blocks over up to ATT_MAX_SPLIT workgroups each (down to one 32-row block
+// per run: each run is then one short chain of loads; the decoder step's
+// cross-attention, 47 blocks per head, runs 26 splits instead of 11: 2% per
+// token, 3% at 440 cached rows), merged by k_attn_combine
+#ifndef ATT_SPLIT_MINBLK
+#define ATT_SPLIT_MINBLK 1
+#endif
+inline int attn_nsplit(size_t groups, size_t nblk) {
+  if (groups >= 256 || nblk < 8) return 1;
+  const size_t want = (512 + groups - 1) / groups, most = nblk / ATT_SPLIT_MINBLK;
+  const size_t n = want < most ? want : most;
+  return n < (size_t)ATT_MAX_SPLIT ? (int)n : ATT_MAX_SPLIT;
+}
+
+// Which kernel a call runs.  qt: 32-row query tiles per k_attn_tile workgroup (1
+// or 2), 0: k_attn with its keys in nsplit runs.  rows: K and V are split as
+// they are loaded (at most 64 rows against keys of their own).
+//
+// At most 8 rows run k_attn.  9 to 64 rows run k_attn_tile, where a wavefront's
+// chain of a quarter of the kv blocks is short, else k_attn and its merge:
+//   * splitting K and V itself a chain takes about 2 us and 1.7 per block (9 rows,
+//     6 heads: 7.2 us at 8 kv blocks, 8.6 at 12, 9.8 at 14, 11.3 at 20, 20.9 at
+//     47) and k_attn 8 to 9 at any length (7.9, 7.8, 8.1, 8.1, 9.0): up to
+//     12 blocks;
+//   * from split blocks, about 3 us and 0.7 per block (5.4 at 12, 7.4 at 24, 8.6
+//     at 32, 11.3 at 47) against 7.2, 7.7, 8.1, 8.3: up to 32 blocks, and beyond
+//     them where there are more than 24 (tile, head) pairs, which fill the chip
+//     and make the merge long (64 rows at 47 blocks: 6 heads 12.2 against 9.4, 12
+//     heads 12.3 against 11.5, 20 heads 12.4 against 12.9).
+// 33 to 64 rows, two tiles a head, take at most 12 runs: with one per block the
+// merge reads more than the runs save (64 rows at 47 blocks, 12 heads: 16.5 us
+// with 32 runs, 12.2 with 12; 20 heads 18.0 with 26, 13.9).
+// More rows run k_attn_tile: 64 per workgroup where those fill 3/4 of the 512
+// workgroup places (two per CU), else 32 (k_attn_tile has both sides measured).
+struct AttnRoute {
+  int qt;
+  bool rows;
+  int nsplit;
+};
+constexpr size_t ATT_TILE_ROWS_BLK = 12, ATT_TILE_KV_BLK = 32, ATT_TILE_KV_PAIRS = 24;
+constexpr int ATT_TWO_TILE_RUNS = 12;
+inline AttnRoute attn_route(size_t t_q, size_t t_kv, size_t n_head, bool presplit, int max_split) {
+  const size_t nblk = (t_kv + ATT_KVB - 1) / ATT_KVB, tiles = (t_q + 31) / 32;
+  AttnRoute r{0, !presplit && t_q <= (size_t)ATT_ROWS_MAX, 1};
+  if (t_q <= (size_t)ATT_ROWS_MAX) {
+    int n = attn_nsplit(n_head, nblk);
+    if (n > max_split) n = max_split;
+    if (tiles > 1 && n > ATT_TWO_TILE_RUNS) n = ATT_TWO_TILE_RUNS;
+    const bool runs = presplit ? nblk > ATT_TILE_KV_BLK && tiles * n_head <= ATT_TILE_KV_PAIRS : nblk > ATT_TILE_ROWS_BLK;
+    if (t_q <= (size_t)ATT_STEP_MAX || (runs && n > 1)) {
+      r.nsplit = n;
+      return r;
+    }
+  }
+  r.qt = !r.rows && (t_q + 63) / 64 * n_head >= 384 ? 2 : 1;
+  return r;
+}
 
 // kv index (within a 16-block) stored at position p of the v^T operands: the
 // middle quads swap (an involution)
@@ -575,8 +635,8 @@ __global__ __launch_bounds__(64 * ATT_NK, 2) void k_attn_tile(int t_q, int t_kv,
   }
 }
 
-// Calls of at most 8 query rows, or of at most 64 against many keys of their own
-// (ROWS).  Workgroup (blockIdx.x, blockIdx.y) = (32 query rows, head); wavefront w takes kv
+// Calls of at most 8 query rows, or of at most 64 against many keys
+// (attn_route).  Workgroup (blockIdx.x, blockIdx.y) = (32 query rows, head); wavefront w takes kv
 // blocks w, w + 2, ...; a causal query row i (at absolute position t_kv - t_q
 // + i) sees kv rows up to its position.
 //

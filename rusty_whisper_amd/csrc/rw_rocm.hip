@@ -1077,20 +1077,6 @@ struct AttnLayout {
   size_t off_kv, off_part, bytes;
 };
 
-// few (query block, head) workgroups -- a decoding step: split the kv
-// blocks over up to ATT_MAX_SPLIT workgroups each (down to one 32-row block
-// per run: each run is then one short chain of loads; the decoder step's
-// cross-attention, 47 blocks per head, runs 26 splits instead of 11: 2% per
-// token, 3% at 440 cached rows), merged by k_attn_combine
-#ifndef ATT_SPLIT_MINBLK
-#define ATT_SPLIT_MINBLK 1
-#endif
-static int attn_nsplit(size_t groups, size_t nblk) {
-  if (groups < 256 && nblk >= 8)
-    return (int)std::min<size_t>(ATT_MAX_SPLIT, std::min<size_t>(nblk / ATT_SPLIT_MINBLK, cdiv(512, groups)));
-  return 1;
-}
-
 // kv_planes = false: the call reads K/V planes split beforehand (the
 // decoder's cross-attention), so the layout holds q's planes and the split
 // runs' partial results only
@@ -1165,36 +1151,28 @@ static int run_attention(const float *q, size_t ldq, const float *k, size_t ldk,
   AttnPlanes P{(uint16_t *)(b + L.off_kv), L.tq_pad, (int)std::min<size_t>(align_up(t_kv, ATT_KVB), L.tkv_pad)};
   if (kv_split) P.kv = kv_split->kv, P.tkv_pad = kv_split->tkv_pad;
   const int nblk = P.tkv_pad / ATT_KVB;
-  const bool rows = !kv_split && t_q <= (size_t)ATT_ROWS_MAX;
-  // 9 to 64 query rows against many keys of their own: k_attn's kv split over
-  // workgroups and its merge (20 rows against 1500, 20 heads: 11.7 us, where
-  // k_attn_tile's chain of 12 blocks per wavefront takes 21.9; against 448 keys
-  // 11.8 and 10.2)
-  const bool long_rows = rows && cdiv(t_kv, ATT_KVB) > (size_t)ATT_TILE_ROWS_BLK;
-  if (t_q > (size_t)ATT_STEP_MAX && !long_rows) {
-    if (!kv_split && !rows)
+  // (the layout's split is for its longest kv; the rule grows with the kv
+  // length, so this call's fits the layout's part buffer)
+  const AttnRoute r = attn_route(t_q, t_kv, (size_t)n_head, kv_split != nullptr, L.nsplit);
+  if (r.qt) {
+    if (!kv_split && !r.rows)
       RW_TRY(launch_attn_split(k, ldk, v, ldv, t_kv, n_head, (uint16_t *)(b + L.off_kv), nblk, s));
-    // 64 query rows per workgroup where those fill 3/4 of the 512 workgroup
-    // places (two per CU), else 32 (k_attn_tile has both sides measured)
-    const bool two = !rows && cdiv(t_q, 64) * (size_t)n_head >= 384;
-    const int nqb = (int)cdiv(t_q, two ? 64 : 32), total = nqb * n_head;
+    const int nqb = (int)cdiv(t_q, 32 * r.qt), total = nqb * n_head;
 #define RW_ATT_TILE(QT, ROWS)                                                                                      \
   hipLaunchKernelGGL((k_attn_tile<QT, ROWS>), dim3((unsigned)total), dim3(64 * ATT_NK), 0, s, (int)t_q, (int)t_kv, \
                      causal, nqb, total, q, (int)ldq, P.kv, nblk, out, (int)ldo, k, (int)ldk, v, (int)ldv)
-    if (rows) RW_ATT_TILE(1, true);
-    else if (two) RW_ATT_TILE(2, false);
+    if (r.rows) RW_ATT_TILE(1, true);
+    else if (r.qt == 2) RW_ATT_TILE(2, false);
     else RW_ATT_TILE(1, false);
 #undef RW_ATT_TILE
     LAUNCH_TRY("k_attn_tile");
     return RW_OK;
   }
-  // this call's split (the layout's is for its longest kv; the rule grows
-  // with the kv length, so this one fits the layout's part buffer)
-  const int nsplit = std::min(L.nsplit, attn_nsplit((size_t)n_head, cdiv(t_kv, ATT_KVB)));
+  const int nsplit = r.nsplit;
   float *part = nsplit > 1 ? (float *)(b + L.off_part) : nullptr;
   const dim3 grid((unsigned)cdiv(t_q, 32), (unsigned)n_head, (unsigned)nsplit);
   const int gw = (causal ? 1 : 0) | nsplit << 1 | n_head << 8;  // k_attn's packed grid
-  if (rows)
+  if (r.rows)
     hipLaunchKernelGGL((k_attn<true>), grid, dim3(128), 0, s, (int)t_q, (int)t_kv, gw, (int)grid.x, q, (int)ldq, k, (int)ldk, v,
                        (int)ldv, out, (int)ldo, part, P, nullptr, 0, BeamCaches{});
   else

@@ -1,7 +1,7 @@
 """Edges of the attention kernels' dispatch (rw_attn.hpp, run_attention): at
-most 8 query rows, or 64 against over 640 keys of their own (k_attn), 9 to 64
-rows (k_attn_tile splitting K and V itself), more (from split blocks), 32 or 64 query rows per workgroup; and
-scores that move the softmax's reference exponent in every block.
+most 8 query rows, or 64 against over 384 keys of their own (k_attn), 9 to 64
+rows (k_attn_tile splitting K and V itself), more (from split blocks), 32 or 64
+query rows per workgroup; and scores that move the softmax's reference.
 
 Bar: 1e-5 of the row's L2 norm against the float64 oracle (operands keep 22
 bits, sums are f32: a few 2^-22 over scores of magnitude s, times s)."""
@@ -28,7 +28,8 @@ def err(got, q, k, v, heads, causal):
 @pytest.mark.parametrize("t_q,t_kv,heads,causal", [
     (8, 33, 2, True), (9, 9, 2, True), (9, 31, 2, False), (32, 129, 1, True), (33, 33, 2, True), (64, 97, 2, True),
     (65, 65, 2, True), (65, 160, 3, False), (1030, 70, 24, False), (1030, 1030, 24, True), (9, 640, 2, True),
-    (9, 641, 2, True), (33, 641, 3, False), (64, 1500, 2, True), (65, 1500, 2, False)], ids=str)
+    (9, 641, 2, True), (33, 641, 3, False), (64, 1500, 2, True), (65, 1500, 2, False), (9, 384, 2, True),
+    (9, 385, 2, True), (32, 385, 3, False), (33, 385, 3, False), (64, 1500, 20, False)], ids=str)
 def test_dispatch_edges(t_q, t_kv, heads, causal):
     rng = np.random.default_rng(t_q + t_kv)
     q, k, v = (rng.standard_normal((t, 64 * heads)).astype(np.float32) for t in (t_q, t_kv, t_kv))

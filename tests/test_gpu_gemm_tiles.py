@@ -61,3 +61,18 @@ def test_cross_attention_operands(torch, n_audio, mixed):  # noqa: F811
     o = OD(p, heads, enc)
     for toks in ([1, 2, 3], [4], list(range(9))):
         assert rel(step(torch, d, toks, n), o.forward_hidden(toks)) <= 4e-3
+
+
+@pytest.mark.parametrize("tokens", [9, 33, 64])
+@pytest.mark.parametrize("n_audio", [1024, 1025, 1500])
+def test_cross_attention_of_short_prompts(torch, n_audio, tokens):  # noqa: F811
+    """Prompts of 9 to 64 tokens against a window whose kept blocks they read in one
+    chain per wavefront (up to 1024 rows) or in runs, against the decoder's bar."""
+    n, heads = 128, 2
+    p = decoder_params(n=n, f=2 * n, n_layer=1, n_vocab=100, n_ctx=80, dtype=8, seed=n_audio + tokens)
+    enc = np.random.default_rng(n_audio).standard_normal((n_audio, n)).astype(np.float32)
+    d = device_decoder(torch, p, heads, n_audio)
+    d.set_audio(torch.from_numpy(enc).to("cuda:0"))
+    o = OD(p, heads, enc)
+    for toks in ([t % 100 for t in range(tokens)], [4]):
+        assert rel(step(torch, d, toks, n), o.forward_hidden(toks)) <= 4e-3
