@@ -38,3 +38,29 @@ def test_sizes_match_the_device_entry(m):
         t.join()
     for i, g in enumerate(got):
         assert np.array_equal(g.view(np.uint32), (want[::-1] if i % 2 else want).view(np.uint32)), i
+
+
+def test_pinned_results():
+    """A pinned result array is written by the device itself: the same bits, and in
+    about half the time of a pageable one of 64 MB (52 against 20 GB/s; the bar,
+    the better of 5 calls each, leaves a quarter of it)."""
+    import time
+
+    import torch
+
+    A.init(0)
+    m, n, k = 1024, 16384, 32
+    rng = np.random.default_rng(1)
+    w = A.DeviceWeight(8, n, k, O.quantize(8, rng.standard_normal((n, k)).astype(np.float32)))
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    outs = [np.zeros((m, n), np.float32), torch.zeros(m, n, pin_memory=True).numpy()]
+    best = []
+    for out in outs:
+        times = []
+        for _ in range(6):
+            t0 = time.perf_counter()
+            A.check(A.lib().rw_rocm_matmul_t_q(w.handle, a.ctypes.data, m, k, None, out.ctypes.data))
+            times.append(time.perf_counter() - t0)
+        best.append(min(times[1:]))
+    assert np.array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
+    assert best[1] <= 0.75 * best[0], best
