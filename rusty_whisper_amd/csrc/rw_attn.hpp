@@ -64,7 +64,7 @@ static_assert(ATT_MAX_SPLIT < 128, "k_attn packs the run count into 7 bits");
 #define ATT_SPLIT_MINBLK 1
 #endif
 inline int attn_nsplit(size_t groups, size_t nblk) {
-  if (groups >= 256 || nblk < 8) return 1;
+  if (groups == 0 || groups >= 256 || nblk < 8) return 1;
   const size_t want = (512 + groups - 1) / groups, most = nblk / ATT_SPLIT_MINBLK;
   const size_t n = want < most ? want : most;
   return n < (size_t)ATT_MAX_SPLIT ? (int)n : ATT_MAX_SPLIT;

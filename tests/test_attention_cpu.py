@@ -2,6 +2,9 @@
 HIP call): the reference's conditions (src/encoder.rs:48-58, 109-119) and
 the kernel's own limits come back as RW_EINVAL with a message."""
 import ctypes as C
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -60,3 +63,14 @@ def test_workspace_size_covers_the_planes():
     # q pairs over 64-row padding, k and v^T pairs over 32-row padding
     n = A.attention_workspace_size(1500, 1500, 1280)
     assert n >= 20 * 1536 * 64 * 4 + 2 * 20 * 1504 * 64 * 4
+
+
+@pytest.mark.parametrize("args", [(0, 1500, 1280), (4, 1500, 32), (1500, 0, 384), (0, 0, 0)])
+def test_workspace_size_of_an_empty_call(args):
+    """No query rows or no head: a size, and no division by their product.  (In a
+    process of its own, which such a division would end.)"""
+    code = f"from rusty_whisper_amd import _abi as A; print(A.attention_workspace_size{args})"
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120,
+                       cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+    assert r.returncode == 0, (r.returncode, r.stderr)
+    assert int(r.stdout.split()[-1]) >= 0
