@@ -1082,29 +1082,37 @@ static int check_matmul_args(const rw_weight *w, const void *a, size_t m, size_t
 
 // ------------------------------------------------------ attention
 
-// Workspace of one attention call: the f16 pairs of q, k and v^T.
+// Workspace of one attention call: the operand blocks of K and v^T (kv: the call
+// or its caller's products write them), and the split runs' partial results of a
+// call of at most 64 rows.
 struct AttnLayout {
   int n_head, tq_pad, tkv_pad, nsplit;
   size_t off_kv, off_part, bytes;
 };
-
-// kv_planes = false: the call reads K/V planes split beforehand (the
-// decoder's cross-attention), so the layout holds q's planes and the split
-// runs' partial results only
-static AttnLayout attn_layout(size_t t_q, size_t t_kv, size_t n_state, bool kv_planes = true) {
+static AttnLayout attn_layout(size_t t_q, size_t t_kv, size_t n_state, bool kv) {
   AttnLayout L{};
   L.n_head = (int)(n_state / ATT_DH);
   L.tq_pad = (int)align_up(t_q, ATT_QB);
   L.tkv_pad = (int)align_up(t_kv, ATT_KVB);
-  // (the size still counts room for q's pairs, as callers were told; q is
-  // split in registers)
-  L.off_kv = align_up(2 * (size_t)L.n_head * L.tq_pad * ATT_DH * 2, 256);
-  const size_t kv = kv_planes ? (size_t)L.n_head * (L.tkv_pad / ATT_KVB) * ATT_BLK * 2 : 0;
-  L.nsplit = attn_nsplit((size_t)(L.tq_pad / ATT_QB) * L.n_head, cdiv(t_kv, ATT_KVB));
-  L.off_part = align_up(L.off_kv + kv, 256);
+  L.nsplit = t_q <= (size_t)ATT_ROWS_MAX ? attn_nsplit((size_t)L.n_head, cdiv(t_kv, ATT_KVB)) : 1;
+  L.off_kv = 0;
+  L.off_part = kv ? align_up((size_t)L.n_head * (L.tkv_pad / ATT_KVB) * ATT_BLK * 2, 256) : 0;
   const size_t part = L.nsplit > 1 ? (size_t)L.nsplit * L.n_head * L.tq_pad * (ATT_DH + 2) * 4 : 0;
   L.bytes = align_up(L.off_part + part, 256);
   return L;
+}
+// a call on f32 rows: more than 64 query rows read blocks
+static AttnLayout attn_call_layout(size_t t_q, size_t t_kv, size_t n_state) {
+  return attn_layout(t_q, t_kv, n_state, t_q > (size_t)ATT_ROWS_MAX);
+}
+// What callers are told to bring: also room for f16 pairs of q, and the blocks
+// and partial results of any route, so that the number they keep stays enough
+// whichever of them a call uses.
+static size_t attn_told_bytes(size_t t_q, size_t t_kv, size_t n_state) {
+  const size_t heads = n_state / ATT_DH, tq_pad = align_up(t_q, ATT_QB), nblk = cdiv(t_kv, ATT_KVB);
+  const size_t nsplit = (size_t)attn_nsplit(tq_pad / ATT_QB * heads, nblk);
+  const size_t q = align_up(heads * tq_pad * ATT_DH * 4, 256), kv = align_up(heads * nblk * ATT_BLK * 2, 256);
+  return align_up(q + kv + (nsplit > 1 ? nsplit * heads * tq_pad * (ATT_DH + 2) * 4 : 0), 256);
 }
 
 // The reference's conditions (src/encoder.rs:48-58, 109-119) plus this
@@ -1275,8 +1283,8 @@ struct DecScratch {
 static DecScratch dec_scratch(const rw_decoder *d, size_t n_tok, bool beams = false) {
   DecScratch S{};
   const size_t row = n_tok * d->n * 4;
-  S.self_att = beams ? attn_layout(1, d->p.n_ctx, n_tok * d->n) : attn_layout(n_tok, d->p.n_ctx, d->n);
-  S.cross_att = attn_layout(n_tok, d->n_audio, d->n, false);  // K/V: the window's kept planes
+  S.self_att = beams ? attn_call_layout(1, d->p.n_ctx, n_tok * d->n) : attn_call_layout(n_tok, d->p.n_ctx, d->n);
+  S.cross_att = attn_layout(n_tok, d->n_audio, d->n, false);  // K/V: the window's kept blocks
   S.off_tok = 0;
   S.off_x = align_up(n_tok * 4, 256);
   S.off_cur = align_up(S.off_x + row, 256);
@@ -1449,7 +1457,7 @@ static LayerLayout layer_layout(size_t n, size_t f, size_t t) {
   L.n = n;
   L.f = f;
   L.act = act_layout(t, std::max(n, f));
-  L.att = attn_layout(t, t, n);
+  L.att = attn_layout(t, t, n, true);  // (its K and V products write the blocks)
   const size_t row = t * n * 4;
   L.off_act = 0;
   L.off_q = align_up(L.act.bytes, 256);
@@ -2134,7 +2142,7 @@ int rw_rocm_block_dots(const rw_weight *w, const int8_t *qa, size_t m, int32_t *
 }
 
 size_t rw_rocm_attention_workspace_size(size_t t_q, size_t t_kv, size_t n_state) {
-  return attn_layout(t_q, t_kv, n_state).bytes;
+  return attn_told_bytes(t_q, t_kv, n_state);
 }
 
 int rw_rocm_attention_dev(const float *q, size_t ldq, const float *k, size_t ldk, const float *v, size_t ldv,
@@ -2146,11 +2154,12 @@ int rw_rocm_attention_dev(const float *q, size_t ldq, const float *k, size_t ldk
   int dev;
   rc = current_device(&dev);
   if (rc) return rc;
-  const AttnLayout L = attn_layout(t_q, t_kv, n_state);
+  const AttnLayout L = attn_call_layout(t_q, t_kv, n_state);
   void *ws = workspace;
   WsHold hold;
   if (ws) {
-    if (workspace_len < L.bytes) return fail(RW_EINVAL, "workspace of %zu bytes < %zu needed", workspace_len, L.bytes);
+    const size_t need = attn_told_bytes(t_q, t_kv, n_state);
+    if (workspace_len < need) return fail(RW_EINVAL, "workspace of %zu bytes < %zu needed", workspace_len, need);
   } else {
     rc = stream_workspace(dev, stream, L.bytes, hold, &ws);
     if (rc) return rc;
@@ -2170,7 +2179,7 @@ int rw_rocm_attention(const float *q, const float *k, const float *v, size_t t_q
   rc = ctx_acquire(dev, &g.c);
   if (rc) return rc;
   Ctx *c = g.c;
-  const AttnLayout L = attn_layout(t_q, t_kv, n_state);
+  const AttnLayout L = attn_call_layout(t_q, t_kv, n_state);
   const size_t off_q = align_up(L.bytes, 256);
   const size_t off_k = align_up(off_q + t_q * n_state * 4, 256);
   const size_t off_v = align_up(off_k + t_kv * n_state * 4, 256);
@@ -2253,8 +2262,10 @@ int rw_rocm_decoder_set_audio_dev(rw_decoder *d, const float *enc_out, void *str
   HIP_TRY(hipSetDevice(d->device));
   hipStream_t s = (hipStream_t)stream;
   const size_t T = d->n_audio, n = d->n;
-  // k and v f32 for one layer, the activation workspace, then splitting
-  const size_t off_k = 0, off_v = align_up(T * n * 4, 256), off_act = align_up(off_v + T * n * 4, 256);
+  // the activation workspace; for at most 8 rows, whose products are GEMVs, one
+  // layer's k and v in f32 before it (more rows' products write the operands)
+  const size_t rows = T <= (size_t)GEMV_MAX_M ? align_up(T * n * 4, 256) : 0;
+  const size_t off_k = 0, off_v = rows, off_act = 2 * rows;
   const size_t bytes = align_up(off_act + act_layout(T, n).bytes, 256);
   int rc = dec_reserve(d, bytes);
   if (rc) return rc;

@@ -137,3 +137,13 @@ def test_fused_mlp_quantization_is_bitwise_the_separate_one(torch, t, n, dtype, 
             os.environ.pop("RW_ENCODER_MLP", None)
         outs.append(xd.cpu().numpy())
     assert np.array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
+
+
+def test_workspace_holds_what_the_layer_uses(torch):
+    """The quantized activations, q, the attention's rows and fc1's, and K and v^T
+    as operand blocks: no f32 rows of K and V, no pairs of q, no kv split."""
+    for t, n in ((1500, 384), (749, 128)):
+        p, dev = build(torch, n, 4 * n, 8, seed=n)
+        uses = (A.workspace_size(t, 4 * n) + 4 * t * (n + n + 4 * n)
+                + n // 64 * ((t + 31) // 32) * 4 * 4 * 64 * 8 * 2)
+        assert uses <= A.EncoderLayer(n // 64, **dev).workspace_size(t) <= uses + 8 * 256
