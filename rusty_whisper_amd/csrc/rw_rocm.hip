@@ -2262,10 +2262,12 @@ int rw_rocm_decoder_set_audio_dev(rw_decoder *d, const float *enc_out, void *str
   HIP_TRY(hipSetDevice(d->device));
   hipStream_t s = (hipStream_t)stream;
   const size_t T = d->n_audio, n = d->n;
-  // the activation workspace; for at most 8 rows, whose products are GEMVs, one
-  // layer's k and v in f32 before it (more rows' products write the operands)
-  const size_t rows = T <= (size_t)GEMV_MAX_M ? align_up(T * n * 4, 256) : 0;
-  const size_t off_k = 0, off_v = rows, off_act = 2 * rows;
+  // one layer's k and v in f32 (at most 8 rows, whose products are GEMVs; more
+  // rows' products write the operands), the activation workspace.  The rows are
+  // kept at any size: the window's prompt and steps take their scratch from the
+  // same allocation, and one that only set_audio fits made the first prompt
+  // free and allocate it again (390 -> 700 us for 4 tokens)
+  const size_t off_k = 0, off_v = align_up(T * n * 4, 256), off_act = align_up(off_v + T * n * 4, 256);
   const size_t bytes = align_up(off_act + act_layout(T, n).bytes, 256);
   int rc = dec_reserve(d, bytes);
   if (rc) return rc;
