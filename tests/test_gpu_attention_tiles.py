@@ -49,14 +49,31 @@ def test_rows_do_not_depend_on_the_tile():
 @pytest.mark.parametrize("t_q", [8, 40, 1030])
 @pytest.mark.parametrize("step", [6.0, -6.0, 40.0])
 def test_moving_maxima(t_q, step):
-    """Scores that rise (or fall) by `step` per key, over blocks of every
-    wavefront: each new block moves the reference exponent, or none does."""
+    """Scores that rise (or fall) so steeply that whatever came before a block (or
+    comes after it) weighs nothing: rescale factors and weights of exactly 0."""
     heads, t_kv = 24, 140
     rng = np.random.default_rng(int(step) + t_q)
     q = np.zeros((t_q, 64 * heads), np.float32)
     k = (rng.standard_normal((t_kv, 64 * heads)) * 0.1).astype(np.float32)
     v = rng.standard_normal((t_kv, 64 * heads)).astype(np.float32)
     q[:, ::64] = 8.0  # score = the key's first value
+    k[:, ::64] = (step * np.arange(t_kv, dtype=np.float32))[:, None]
+    assert err(A.attention(q, k, v, heads, False), q, k, v, heads, False) <= 1e-5
+
+
+@pytest.mark.parametrize("t_q", [8, 40, 100, 1030])
+@pytest.mark.parametrize("step", [0.03, 0.06])
+def test_rescales_that_matter(t_q, step):
+    """Scores that rise by 4 or 8 nats over the 128 keys between a wavefront's
+    blocks, in some query rows and not in others (12 blocks: two rescales each):
+    what came before keeps a weight of 2^-6 or 2^-11, far above the bar."""
+    heads, t_kv = 24, 384
+    rng = np.random.default_rng(int(100 * step) + t_q)
+    q = np.zeros((t_q, 64 * heads), np.float32)
+    k = (rng.standard_normal((t_kv, 64 * heads)) * 0.1).astype(np.float32)
+    v = rng.standard_normal((t_kv, 64 * heads)).astype(np.float32)
+    slope = rng.choice(np.array([1.0, 0.9, 0.0, -1.0], np.float32), (t_q, heads))
+    q[:, ::64] = 8.0 * slope  # score = slope x the key's first value
     k[:, ::64] = (step * np.arange(t_kv, dtype=np.float32))[:, None]
     assert err(A.attention(q, k, v, heads, False), q, k, v, heads, False) <= 1e-5
 
