@@ -940,7 +940,7 @@ def main() -> int:
             "limiter": "operand delivery at one wavefront per SIMD (the k loop takes the MFMA-only loop plus "
                        "35-50% of the loads-only one), and every wavefront waiting for its first blocks and "
                        "storing its tile at once: MFMA busy about a quarter of the kernel's time, L2->CU operand "
-                       "traffic 10-25x the unique bytes (rocprofv3 counters in "
+                       "traffic 16-19x the unique bytes (rocprofv3 counters in "
                        "profiles/k_gemm_q5_1_large_v3_encoder_m1500.md)",
             "avg_launch_us": round(gemm_ms * 1e3, 2),
             "launch_us_by_launch": per_shape,

@@ -23,7 +23,7 @@
 // ones keep their f16 bits: a step of 2^-24 is 2^-36 of the largest.
 // Inputs must stay below f16's 65504 in magnitude (whisper's projections are
 // far below it); inputs below about 1e-3 lose a few bits to f16 subnormal
-// residuals.  The softmax is online (running reference exponent and sum per
+// residuals.  The softmax is online (running reference score and sum per
 // query row) in f32, which is the reference's max / exp / sum / divide
 // reordered.
 //
@@ -170,7 +170,9 @@ __device__ inline AttSplit8 att_split8(const float (&v)[8]) {
 // its 8 rows' value, 128-byte runs of a row per load; 1 KB runs written).
 // Rows >= t_kv are zeros.  Bound by its bytes, 8 t n read and 8 t n written:
 // 4.9 us for large-v3's 30.7 MB (7.1 us when v^T went through LDS to row-major
-// planes).
+// planes).  Into blocks that the call before has just read it takes 12, likely
+// because other XCDs' L2s still hold the lines it stores to (attention calls that
+// take turns over 8 workspaces 45 us each, over one 52).
 __global__ __launch_bounds__(256) void k_attn_split(const float *__restrict__ k, int ldk, const float *__restrict__ v,
                                                     int ldv, int t_kv, int nblk, uint16_t *__restrict__ kv) {
   const int head = blockIdx.x / nblk, blk = blockIdx.x % nblk, t = threadIdx.x;
@@ -439,12 +441,13 @@ __device__ inline void att_load_q(const float *__restrict__ qf, int ldq, int row
 //
 // Bound by the matrix cores' rate under load and the softmax beside it: with
 // loads and softmax taken out, large-v3's layer (20 heads, t = 1500, 35.5
-// GFLOP of f16 products) still takes 31 us, 1.3 PFLOP/s, of 41 us (two
+// GFLOP of f16 products) still takes 31 us, 1.15 PFLOP/s, of 44 us (two
 // wavefronts of 64 queries per row group pair on 960 wavefronts took 53: one
 // wavefront per SIMD, accumulators moving between register files, 16-byte
 // loads).  QT = 2 keeps q's operands in LDS (232 registers, two wavefronts per
 // SIMD) and loads 16 KB per 48 products; QT = 1 loads the same per 24, so it
-// is for calls that 64-row tiles leave short of workgroups: 20 heads 41 against
+// is for calls that 64-row tiles leave short of workgroups (each pair on one
+// build, before the reference score was subtracted first): 20 heads 41 against
 // 47 us, but 12 heads 34.4 against 32.9, 6 heads at t = 749 12.7 against 8.5,
 // 227 rows against 1500 (20 heads) 21 against 13 us.  Eight wavefronts per
 // workgroup: 46 (QT = 2) and 57 us (QT = 1).

@@ -390,8 +390,8 @@ __device__ inline float dense_finish(const float (&acc)[8], const float *__restr
 // LDS reads; rows 36 floats apart start on distinct banks).
 // Bound by the VALU: a product and a sum rounded apart are two instructions,
 // 2 m n k / 64 of them at 4 cycles each: 125 us at 2.4 GHz for 1500 x 1280 x
-// 1280 (147 us; R = 2 with 4-byte LDS reads, two per product, took 268; R = 4
-// 149, at two wavefronts per SIMD).  R = 1 is for launches that 32-row tiles
+// 1280 (130 us; 4-byte LDS reads, two per product, took 256; R = 4 measured 149
+// where R = 2 measured 147, at two wavefronts per SIMD).  R = 1 is for launches that 32-row tiles
 // leave under 512 workgroups: 100 x 384 x 1536 21 against 55 us, 224 x 1280 x
 // 1280 39 against 49, but 1500 x 384 x 384 (564 tiles) 21.5 against 20.8.  VEC:
 // rows start on 16 bytes.
