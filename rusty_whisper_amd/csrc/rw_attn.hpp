@@ -144,7 +144,7 @@ typedef float att_v16f __attribute__((ext_vector_type(16)));
 typedef float att_v2f __attribute__((ext_vector_type(2)));
 typedef _Float16 att_v2h __attribute__((ext_vector_type(2)));
 constexpr float ATT_LOG2E = 1.4426950408889634f;
-constexpr float ATT_STEP_PS = 4096.0f;  // k_attn's scale of P
+constexpr float ATT_PS = 4096.0f;  // P's scale in its products
 
 // x = hi + lo, both f16
 __device__ inline void att_split(float x, uint16_t &hi, uint16_t &lo) {
@@ -327,21 +327,24 @@ __device__ inline void att_split_v(const AttVRaw &x, AttV &o) {
 }
 
 // The softmax's running state of one query (a lane pair (n, n + 32) holds one):
-// m, a reference score, and lsum, this lane's sum of p = 2^(log2(e) (s - m) +
-// ATT_PS).  m is the largest score seen when it was set, and moved only when a
-// score passes it by more than ATT_SLACK (3.9 bits: p <= 2^15.9 fits f16): then
-// the output and the sum are rescaled.  Any m gives the same quotient; p >= 2^12
-// at the row's maximum is what keeps small probabilities' f16 bits (hi + lo hold
-// 2^-24 absolute, 2^-36 of the maximum): where a row's mass is on one key of
-// little value, its output is made of probabilities far below the maximum, and
-// with p = 2^8 there its error was 16 times larger (a gap of 2^20: up to 4e-5 of
-// the row).  s - m comes before the factor, as a score's difference from one near
-// it is exact: with log2(e) m rounded on its own, scores past 2^26 (|q|, |k| in
-// the thousands) left every p at infinity or 0 (one instruction less per score,
-// 43.6 against 44.0 us at 20 heads and t = 1500).  Rescaling at every new maximum
-// moved some query of a tile in nearly every block (a wavefront sees 12 of them
-// at t = 1500); with 3.9 bits of slack it is a few of them.
-constexpr float ATT_PS = 12.0f, ATT_SLACK = 3.9f / ATT_LOG2E;
+// m, a reference score, and lsum, this lane's sum of p = 2^(log2(e) (s - m)).  m
+// is the largest score seen when it was set, and moved only when a score passes it
+// by more than ATT_SLACK (3.9 bits: ATT_PS p <= 2^15.9 fits f16): then the output
+// and the sum are rescaled.  Any m gives the same quotient; ATT_PS p >= 2^12 at
+// the row's maximum is what keeps small probabilities' f16 bits (hi + lo hold
+// 2^-24 absolute, 2^-36 of the maximum): where a row's mass is on one key of little
+// value, its output is made of probabilities far below the maximum, and with 2^8
+// there its error was 16 times larger (a gap of 2^20: up to 4e-5 of the row).  The
+// scale is a product and not 12 in the exponent, whose rounding near 12 is 2^-21 of
+// every probability: rows of little spread, sums that cancel, came out at 2.2e-7 of
+// their norm (100 keys; 1.2e-7 now).  s - m comes before log2(e), as a score's
+// difference from one near it is exact: with log2(e) m rounded on its own, scores
+// past 2^26 (|q|, |k| in the thousands) left every p at infinity or 0.  (20 heads
+// at t = 1500: 42.9 us with 2^8 and log2(e) s - log2(e) m, 44.8 with the difference
+// first and 12 in the exponent, 45.5 so.)  Rescaling at every new maximum moved
+// some query of a tile in nearly every block (a wavefront sees 12 of them at t =
+// 1500); with 3.9 bits of slack it is a few of them.
+constexpr float ATT_SLACK = 3.9f / ATT_LOG2E;
 constexpr float ATT_NONE = -1e30f;  // no score seen yet
 
 // the largest score of the query's 32 kv rows (s: lane (h, n) holds query n's
@@ -367,12 +370,15 @@ __device__ inline void att_rescale(float mx, float &m, float &lsum, att_v16f (&o
   o[1] *= alpha;
   m = mnew;
 }
-// p - hi, one mixed-precision FMA each (the compiler converts and subtracts)
+// ATT_PS p - hi, one mixed-precision FMA each (the compiler multiplies, converts
+// and subtracts).  hi comes from two instructions behind the exponential, so the
+// wait state that its consumers need, and that the compiler does not see here, has
+// passed.
 __device__ inline att_v2f att_resid(att_v2f p, att_v2h hi) {
   att_v2f r;
   const uint32_t hb = __builtin_bit_cast(uint32_t, hi);
-  asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r.x) : "v"(hb), "v"(p.x));
-  asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r.y) : "v"(hb), "v"(p.y));
+  asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel_hi:[0,0,1]" : "=v"(r.x) : "v"(p.x), "s"(ATT_PS), "v"(hb));
+  asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "=v"(r.y) : "v"(p.y), "s"(ATT_PS), "v"(hb));
   return r;
 }
 // scores to the P^T operands; their sum to lsum
@@ -380,11 +386,13 @@ __device__ inline void att_probs(const att_v16f &s, float m, float &lsum, att_v8
   float s0 = 0.0f, s1 = 0.0f;
 #pragma unroll
   for (int i = 0; i < 16; i += 2) {
-    const att_v2f p = {__builtin_amdgcn_exp2f(__builtin_fmaf(s[i] - m, ATT_LOG2E, ATT_PS)),
-                       __builtin_amdgcn_exp2f(__builtin_fmaf(s[i + 1] - m, ATT_LOG2E, ATT_PS))};
+    const att_v2f p = {__builtin_amdgcn_exp2f((s[i] - m) * ATT_LOG2E),
+                       __builtin_amdgcn_exp2f((s[i + 1] - m) * ATT_LOG2E)};
     s0 += p.x;
     s1 += p.y;
-    const att_v2h hi = __builtin_convertvector(p, att_v2h);  // one packed conversion
+    // f16(p) times ATT_PS, a packed conversion and product: what f16 drops of a p
+    // below 2^-14 is in the residual
+    const att_v2h hi = __builtin_convertvector(p, att_v2h) * (_Float16)ATT_PS;
     const att_v2f r = att_resid(p, hi);
     const att_v2h lo = __builtin_convertvector(r, att_v2h);
     ph[i >> 3][i & 7] = hi.x, ph[i >> 3][(i & 7) + 1] = hi.y;
@@ -441,7 +449,7 @@ __device__ inline void att_load_q(const float *__restrict__ qf, int ldq, int row
 //
 // Bound by the matrix cores' rate under load and the softmax beside it: with
 // loads and softmax taken out, large-v3's layer (20 heads, t = 1500, 35.5
-// GFLOP of f16 products) still takes 31 us, 1.15 PFLOP/s, of 44 us (two
+// GFLOP of f16 products) still takes 31 us, 1.15 PFLOP/s, of 45 us (two
 // wavefronts of 64 queries per row group pair on 960 wavefronts took 53: one
 // wavefront per SIMD, accumulators moving between register files, 16-byte
 // loads).  QT = 2 keeps q's operands in LDS (232 registers, two wavefronts per
@@ -605,7 +613,7 @@ __global__ __launch_bounds__(64 * ATT_NK, 2) void k_attn_tile(int t_q, int t_kv,
       float den = 0.0f;
 #pragma unroll
       for (int w = 0; w < NK; ++w) den += xl[w][qt * 32 + n] * __builtin_amdgcn_exp2f((xm[w][qt * 32 + n] - mu) * ATT_LOG2E);
-      xinv[qt * 32 + n] = 1.0f / den;
+      xinv[qt * 32 + n] = 1.0f / (den * ATT_PS);
     }
     const float sc = __builtin_amdgcn_exp2f((m[qt] - mu) * ATT_LOG2E);
     o[qt][0] *= sc;
@@ -756,7 +764,7 @@ __global__ __launch_bounds__(128) void k_attn(int t_q, int t_kv, int gw, int nx,
       ps += p;
       // P enters the products as 2^12 p, so that small probabilities keep
       // their f16 bits; the output is divided by 2^12 lsum at the end
-      const float p12 = p * ATT_STEP_PS;
+      const float p12 = p * ATT_PS;
       const _Float16 ph1 = (_Float16)p12;
       ph[i >> 3][i & 7] = ph1;
       pl[i >> 3][i & 7] = (_Float16)(p12 - (float)ph1);
@@ -795,7 +803,7 @@ __global__ __launch_bounds__(128) void k_attn(int t_q, int t_kv, int gw, int nx,
     const float s0 = __builtin_amdgcn_exp2f((m - mu) * ATT_LOG2E), s1 = __builtin_amdgcn_exp2f((m1 - mu) * ATT_LOG2E);
     float lt = lsum * s0 + l1 * s1;
     lt += __shfl_xor(lt, 32);
-    const float inv = part ? 1.0f : 1.0f / (lt * ATT_STEP_PS);
+    const float inv = part ? 1.0f : 1.0f / (lt * ATT_PS);
     if (part && h == 0 && q0 + n < t_q) {
       const size_t pr = ((size_t)blockIdx.z * gy + head) * P.tq_pad + q0 + n;
       float *pml = part + (size_t)gz * gy * P.tq_pad * ATT_DH;
@@ -884,7 +892,7 @@ __global__ __launch_bounds__(256) void k_attn_combine(const float *__restrict__ 
       den += lz[z] * w;
     }
   }
-  const float y = num / (den * ATT_STEP_PS);
+  const float y = num / (den * ATT_PS);
   out[(size_t)q * ld_out + head * ATT_DH + d] = y;
   if (rec) combine_records(rec, q, head * ATT_DH + d, t_q, y, rec_off);  // whole wavefronts (uniform)
 }

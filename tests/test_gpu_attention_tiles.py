@@ -126,3 +126,20 @@ def test_scores_of_large_operands(t_q, scale):
         best = s == s.max(axis=1, keepdims=True)
         ref = best @ v[:, c].astype(np.float64) / best.sum(axis=1, keepdims=True)
         assert np.max(np.max(np.abs(got[:, c] - ref), axis=1) / np.linalg.norm(ref, axis=1)) <= 1e-6, hd
+
+
+@pytest.mark.parametrize("t_q", [40, 100, 1030])
+def test_rows_of_little_spread(t_q):
+    """Near-equal scores, whose row is a mean that cancels: what is random in each
+    probability stays in it undivided.  The operands' 22 bits (2^-23 at most, 7e-8
+    rms), the output's rounding (4e-8) and a few sums of that size leave 1.2e-7 of
+    the rows' norm; an exponent rounded near 12 instead of near 0 added 1.9e-7
+    (2^-21 / sqrt(3) times ln 2)."""
+    heads, t_kv = 24, 100
+    rng = np.random.default_rng(t_q)
+    q, k, v = (rng.standard_normal((t, 64 * heads)).astype(np.float32) for t in (t_q, t_kv, t_kv))
+    q *= np.float32(0.1)
+    k *= np.float32(0.1)
+    ref = mha(q, k, v, heads, False, dtype=np.float64)
+    got = A.attention(q, k, v, heads, False).astype(np.float64)
+    assert np.linalg.norm(got - ref) <= 1.7e-7 * np.linalg.norm(ref)
