@@ -172,7 +172,7 @@ __device__ inline AttSplit8 att_split8(const float (&v)[8]) {
 // 4.9 us for large-v3's 30.7 MB (7.1 us when v^T went through LDS to row-major
 // planes).  Into blocks that the call before has just read it takes 12, likely
 // because other XCDs' L2s still hold the lines it stores to (attention calls that
-// take turns over 8 workspaces 45 us each, over one 52).
+// take turns over 8 workspaces 48 us each, over one 55).
 __global__ __launch_bounds__(256) void k_attn_split(const float *__restrict__ k, int ldk, const float *__restrict__ v,
                                                     int ldv, int t_kv, int nblk, uint16_t *__restrict__ kv) {
   const int head = blockIdx.x / nblk, blk = blockIdx.x % nblk, t = threadIdx.x;
