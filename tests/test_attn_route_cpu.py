@@ -8,6 +8,8 @@ import subprocess
 
 import pytest
 
+from rusty_whisper_amd import _abi as A
+
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(os.path.dirname(HERE), "rusty_whisper_amd", "csrc")
 
@@ -66,3 +68,15 @@ def test_takes_the_faster_kernel(route, t_q, t_kv, heads, presplit, tile, split)
 ])
 def test_lines(route, t_q, t_kv, heads, presplit, want):
     assert route(t_q, t_kv, heads, presplit) == want
+
+
+@pytest.mark.parametrize("heads", [1, 6, 20, 300])
+def test_workspace_holds_what_the_route_uses(route, heads):
+    """K and v^T as operand blocks (16 KB per head and 32 keys), or the runs' partial
+    results (64 rows of 64 values, a maximum and a sum per run and head)."""
+    for t_q in (1, 8, 9, 32, 33, 64, 65, 1500):
+        for t_kv in (1, 255, 256, 384, 385, 1500):
+            qt, rows, nsplit = route(t_q, t_kv, heads, False)
+            blocks = heads * ((t_kv + 31) // 32) * 16384 if qt and not rows else 0
+            parts = nsplit * heads * 64 * 66 * 4 if nsplit > 1 else 0
+            assert A.attention_workspace_size(t_q, t_kv, 64 * heads) >= blocks + parts, (t_q, t_kv)
